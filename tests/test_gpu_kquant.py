@@ -45,6 +45,22 @@ def test_kquant_dequant_bit_exact(gpu, orc, t, n):
 
 
 @pytest.mark.parametrize("t", [Q4_K, Q6_K])
+@pytest.mark.parametrize("off", [0, 4])
+@pytest.mark.parametrize("blocks,tail", [(8192, 0), (8193, 0), (16384, 0), (16385, -3), (24577, -1)])
+def test_kquant_dequant_passes(gpu, orc, t, off, blocks, tail):
+    """Around the blocks of one and two passes of the whole grid (256 CUs x 8
+    workgroups x 4 wavefronts), with partial last blocks and quads; blocks of
+    all byte values, data and output 16-byte aligned or 4 bytes past it."""
+    n = 256 * blocks + tail
+    data = np.random.default_rng(blocks + t).integers(0, 256, blocks * TS[t], dtype=np.uint8)
+    db, dp = up(data, offset=off)
+    ob = DeviceBuffer(4 * n + off + 16)
+    ops.dequantize(t, dp, data.nbytes, n, ob.ptr + off)
+    st, ref = orc.dequantize(t, data, n)
+    assert st == 0 and same(down(ob, np.float32, n, off), ref)
+
+
+@pytest.mark.parametrize("t", [Q4_K, Q6_K])
 def test_kquant_dequant_random_bytes_unaligned_out(gpu, orc, t):
     """Every byte random (d / dmin may be NaN, inf or subnormal); output at a
     4-byte (not 16-byte) aligned address."""

@@ -31,22 +31,89 @@ using whd::q6k_quant;
 template <int TYPE>
 constexpr int kq_bytes() { return TYPE == WH_TYPE_Q4_K ? 144 : 210; }
 
-// One thread per quad of 4 consecutive outputs (64 quads per block), grid-stride.
+// Four consecutive outputs per thread and quad (64 quads, one KiB, per block
+// and wavefront).  Bound by the f32 output written (1 KiB against 144 or 210 B
+// read per block), as long as the loads are few and wide: the byte-wise decode
+// of kq_quad took 105 us (Q4_K) and 100 us (Q6_K) for 14336 x 4096; with one
+// 16-byte header load and two quant bytes per quad (Q4_K), or one dword of ql,
+// two bytes of qh, the scale and d (Q6_K), 57 us and 60 us (4.7 TB/s; a fill of
+// that size writes 6.9 TB/s).  Blocks per wavefront and pass: Q4_K two (one: 67 us, four
+// 66 us), Q6_K one (two: 67 us); 8 workgroups per CU (Q4_K with 16: 69 us).
 template <int TYPE>
+constexpr int kq_run() { return TYPE == WH_TYPE_Q4_K ? 2 : 1; }
+
+// Quad c of a block as kq_quad decodes it (same operations in the same order).
+// Q4_K: b 16-byte aligned.
+template <int TYPE>
+__device__ __forceinline__ void kq_quad_wide(const uint8_t* b, int c, float v[4]) {
+  if constexpr (TYPE == WH_TYPE_Q4_K) {
+    const uint4 h = *reinterpret_cast<const uint4*>(b);
+    const uint32_t q = *reinterpret_cast<const uint16_t*>(b + 16 + 2 * c);
+    const float d = whd::f16_bits_to_f32(h.w & 0xFFFFu), dmin = whd::f16_bits_to_f32(h.w >> 16);
+    // scales 2p and 2p + 1 are bits 0..5 and 14..19 of the 24 bits at bit 24p
+    const int p = c >> 4;
+    const uint32_t lo = p == 0 ? h.x : (p == 1 ? (h.x >> 24) | (h.y << 8) : (p == 2 ? (h.y >> 16) | (h.z << 16) : h.z >> 8));
+    const uint32_t s = (lo >> ((c & 8) ? 14 : 0)) & 63u;
+    const float ds = __fmul_rn(d, static_cast<float>(s));
+#pragma unroll
+    for (int t = 0; t < 4; t++) v[t] = __fadd_rn(__fmul_rn(ds, static_cast<float>((q >> (4 * t)) & 15u)), dmin);
+  } else {
+    uint32_t ql;
+    uint16_t qh;
+    __builtin_memcpy(&ql, b + 16 * (c >> 3) + 4 * (c & 3), 4);  // blocks are 2-byte aligned
+    __builtin_memcpy(&qh, b + 128 + c, 2);
+    const float d = whd::f16_bits_to_f32(b16(b + 208)), s = static_cast<float>(b[192 + (c >> 2)]);
+    const float ds = __fmul_rn(d, s);
+    // the two bytes of qh; past the last one (byte 64 is a scale) the bits are 0
+    uint32_t hi = c == 63 ? qh & 0xFFu : qh;
+    if (c >= 32) {
+      ql >>= 4;
+      hi >>= 2;
+    }
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+      const uint32_t q = ((ql >> (8 * t)) & 15u) | (((hi >> (2 * t)) & 3u) << 4);
+      v[t] = __fmul_rn(__fmul_rn(ds, static_cast<float>(static_cast<int>(q) - 32)), 0.015625f);
+    }
+  }
+}
+
+// WIDE: output (and for Q4_K input) 16-byte aligned.
+template <int TYPE, bool WIDE>
 __global__ __launch_bounds__(256) void kq_dequant_kernel(const uint8_t* __restrict__ data, float* __restrict__ out,
                                                          size_t n) {
-  const size_t nquads = (n + 3) / 4;
-  for (size_t qd = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; qd < nquads;
-       qd += static_cast<size_t>(gridDim.x) * blockDim.x) {
-    const size_t blk = qd >> 6;
-    const int c = static_cast<int>(qd & 63);
-    float v[4];
-    kq_quad<TYPE>(data + blk * kq_bytes<TYPE>(), c, v);
-    const size_t e = 4 * qd;
-    if (e + 4 <= n && (reinterpret_cast<uintptr_t>(out) & 15) == 0) {
-      *reinterpret_cast<float4*>(out + e) = make_float4(v[0], v[1], v[2], v[3]);
-    } else {
-      for (int t = 0; t < 4 && e + t < n; t++) out[e + t] = v[t];
+  constexpr int kRun = kq_run<TYPE>();
+  const size_t nblk = (n + 255) / 256;
+  const int lane = static_cast<int>(threadIdx.x) & 63;
+  const size_t waves = static_cast<size_t>(gridDim.x) * (blockDim.x >> 6);
+  const size_t wave = static_cast<size_t>(blockIdx.x) * (blockDim.x >> 6) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // a zero the compiler cannot see through: the block address counts as the
+  // lane's own, so the header comes by vector loads (a scalar load per block
+  // misses the small scalar cache every time)
+  uint32_t lane0 = 0;
+  asm("" : "+v"(lane0));
+  data += lane0;
+  for (size_t b0 = wave; b0 < nblk; b0 += waves * kRun) {
+    if (WIDE && (b0 + (kRun - 1) * waves + 1) * 256 <= n) {
+      float v[kRun][4];
+#pragma unroll
+      for (int u = 0; u < kRun; u++) kq_quad_wide<TYPE>(data + (b0 + u * waves) * kq_bytes<TYPE>(), lane, v[u]);
+#pragma unroll
+      for (int u = 0; u < kRun; u++)
+        *reinterpret_cast<float4*>(out + (b0 + u * waves) * 256 + 4 * lane) =
+            make_float4(v[u][0], v[u][1], v[u][2], v[u][3]);
+      continue;
+    }
+    for (size_t b = b0; b < nblk && b < b0 + kRun * waves; b += waves) {
+      const size_t e = b * 256 + 4 * lane;
+      float v[4];
+      if (WIDE && (b + 1) * 256 <= n) {
+        kq_quad_wide<TYPE>(data + b * kq_bytes<TYPE>(), lane, v);
+        *reinterpret_cast<float4*>(out + e) = make_float4(v[0], v[1], v[2], v[3]);
+      } else {
+        kq_quad<TYPE>(data + b * kq_bytes<TYPE>(), lane, v);
+        for (int t = 0; t < 4 && e + t < n; t++) out[e + t] = v[t];
+      }
     }
   }
 }
@@ -181,9 +248,16 @@ namespace wh {
 int launch_dequantize_kquant(int type, const void* data, size_t n, float* out, hipStream_t s) {
   if (n == 0) return WH_OK;
   const uint8_t* p = static_cast<const uint8_t*>(data);
-  const unsigned grid = kq_grid((n + 3) / 4, 256);
-  if (type == WH_TYPE_Q4_K) kq_dequant_kernel<WH_TYPE_Q4_K><<<grid, 256, 0, s>>>(p, out, n);
-  else kq_dequant_kernel<WH_TYPE_Q6_K><<<grid, 256, 0, s>>>(p, out, n);
+  const size_t wgs = (n + 1023) / 1024, cap = static_cast<size_t>(wh::cu_count()) * 8;  // a block per wavefront
+  const unsigned grid = static_cast<unsigned>(wgs < cap ? wgs : cap);
+  const bool o16 = wh::aligned(out, 16);
+  if (type == WH_TYPE_Q4_K) {
+    if (o16 && wh::aligned(data, 16)) kq_dequant_kernel<WH_TYPE_Q4_K, true><<<grid, 256, 0, s>>>(p, out, n);
+    else kq_dequant_kernel<WH_TYPE_Q4_K, false><<<grid, 256, 0, s>>>(p, out, n);
+  } else {
+    if (o16) kq_dequant_kernel<WH_TYPE_Q6_K, true><<<grid, 256, 0, s>>>(p, out, n);
+    else kq_dequant_kernel<WH_TYPE_Q6_K, false><<<grid, 256, 0, s>>>(p, out, n);
+  }
   WH_LAUNCH_CHECK("dequantize (k-quant) kernel launch");
   return WH_OK;
 }
