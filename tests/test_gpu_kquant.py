@@ -8,7 +8,7 @@ import pytest
 
 from tests._gpu import down, gemv, up
 from tests._oracle import max_abs, rel_l2
-from tests.test_oracle_kquant import np_q4_k, np_q6_k, q4k_block, q6k_block
+from tests.test_oracle_kquant import f16b, np_q4_k, np_q6_k, q4k_block, q6k_block
 from woolly_amd import gguf, ops, synth
 from woolly_amd.device import DeviceBuffer
 
@@ -192,6 +192,52 @@ KQ_MATMUL = [(3, 300, 4096), (8, 1024, 2048), (17, 768, 256), (64, 129, 4096), (
              (257, 384, 1024), (512, 256, 14336)]
 
 
+# every token tile (32, 64, 128), partial tiles, odd row counts (stage records
+# that start 8 bytes off a 16-byte boundary), one super-block per row, and
+# tiles shared by two workgroups of the stream-K grid (14337 and 5000 rows)
+KQ_EDGES = [(17, 1, 256), (32, 255, 256), (33, 257, 768), (64, 301, 512), (65, 513, 2304), (128, 1001, 1024),
+            (129, 14337, 256), (257, 5000, 1280)]
+
+
+@pytest.mark.parametrize("t", [Q4_K, Q6_K])
+@pytest.mark.parametrize("m,n,k", KQ_EDGES)
+def test_kquant_matmul_edges(gpu, orc, t, m, n, k):
+    """Per-output error of about k roundings of f32 sums of the terms' size:
+    rel-L2 <= 2e-6; bfloat16 activations give the widened ones' bits."""
+    print(f"[case] kquant edges type={t} m={m} n={n} k={k}", flush=True)
+    w = synth.quantized_weight(t, n, k, seed=n + k + t)
+    x = synth.activations(m * k, seed=m + t).reshape(m, k)
+    x = (x.view(np.uint32) & np.uint32(0xFFFF0000)).view(np.float32)  # bf16 values
+    got = kq_matmul(t, w, x, m, n, k)
+    rows = sorted({0, m // 2, m - 1})
+    ref = orc.matmul_rows_f64(t, w, n, k, x, m, np.array(rows))
+    assert rel_l2(got[rows], ref) <= 2e-6
+    wb, wp = up(w)
+    xb, xp = up((x.view(np.uint32) >> 16).astype(np.uint16))
+    yb = DeviceBuffer(4 * m * n)
+    wsz = ops.matmul_x_workspace_bytes(t, n, k, m, ops.TYPE_BF16)
+    ws = DeviceBuffer(wsz)
+    ops.quantized_matmul_x(t, wp, w.nbytes, n, k, xp, ops.TYPE_BF16, m, yb.ptr, ws, wsz)
+    assert np.array_equal(down(yb, np.float32, m * n).reshape(m, n), got)
+
+
+@pytest.mark.parametrize("t", [Q4_K, Q6_K])
+def test_kquant_nonfinite_scales(gpu, orc, t):
+    """A block scale d of inf or NaN makes its row NaN, as (d * s) * q does
+    where s or q is 0; the other rows are untouched."""
+    m, n, k = 40, 96, 1024
+    w = synth.quantized_weight(t, n, k, seed=5 + t).reshape(n, -1, TS[t]).copy()
+    x = synth.activations(m * k, seed=6).reshape(m, k)
+    base = kq_matmul(t, w.reshape(-1), x, m, n, k)
+    at = 12 if t == Q4_K else 208
+    w[7, 2, at:at + 2] = f16b(np.inf)
+    w[50, 0, at:at + 2] = f16b(np.nan)
+    got = kq_matmul(t, w.reshape(-1), x, m, n, k)
+    assert np.all(np.isnan(got[:, [7, 50]]))
+    rest = [r for r in range(n) if r not in (7, 50)]
+    assert np.array_equal(got[:, rest], base[:, rest])
+
+
 def kq_matmul(t, w, x, m, n, k, w_offset=0):
     wb, wp = up(w, offset=w_offset)
     xb, xp = up(x)
@@ -227,7 +273,8 @@ def test_kquant_matmul_matches_gemv(gpu, t):
 
 
 @pytest.mark.parametrize("t", [Q4_K, Q6_K])
-@pytest.mark.parametrize("hidden,n_ff,m", [(256, 512, 1), (512, 1024, 4), (4096, 1024, 64), (256, 20480, 5)])
+@pytest.mark.parametrize("hidden,n_ff,m", [(256, 512, 1), (512, 1024, 4), (4096, 1024, 64), (256, 20480, 5),
+                                          (256, 768, 70), (512, 20480, 257), (4096, 14336, 130)])
 def test_kquant_ffn_parity(gpu, orc, t, hidden, n_ff, m):
     """The SwiGLU FFN layer on K-quant weights: decode (fused gate/up GEMV) and
     prefill (RMSNorm and SwiGLU packed into the tiled GEMM's activations, each

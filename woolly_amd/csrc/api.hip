@@ -486,6 +486,9 @@ WH_API int wh_quantized_matmul_x(int type, const void* weights, size_t weight_nb
   if (n_tokens > 16 && wh::is_block_type(type) &&
       wh::gemm_tiled_ok(type, weights, static_cast<const float*>(x), n_rows, k, n_tokens))
     return wh::launch_gemm_tiled_bf16(type, weights, n_rows, k, xb, n_tokens, y, workspace, s);
+  if (n_tokens > 16 && wh::gemm_kquant_ok(type, weights, static_cast<const float*>(x), n_rows, k, n_tokens))
+    return wh::launch_gemm_kquant(type, weights, n_rows, k, static_cast<const float*>(x), n_tokens, y, workspace, s,
+                                  /*xb=*/true);
   // otherwise widen into the workspace and run the f32 product
   float* xf = static_cast<float*>(workspace);
   const size_t head = align_up(n_tokens * k * sizeof(float), 256);

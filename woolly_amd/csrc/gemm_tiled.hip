@@ -32,28 +32,14 @@
 //     conversion, exact), multiplies, and applies the block scale.
 //   Tiles are numbered so that the tiles resident on one XCD share a token
 //     tile, whose activation fragments then stay in that XCD's L2.
-#include "wh_blocks.hpp"
+#include "gemm_dev.hpp"
+#include "gemm_sb_api.hpp"
 
 #include <atomic>
 
-// raw buffer load / store of 16 bytes (llvm.amdgcn.raw.buffer.{load,store}.v4f32)
-__device__ float __attribute__((ext_vector_type(4))) gt_buffer_load_x4(int __attribute__((ext_vector_type(4))) rsrc,
-                                                                       int voffset, int soffset, int aux)
-    __asm("llvm.amdgcn.raw.buffer.load.v4f32");
-__device__ void gt_buffer_store_x4(float __attribute__((ext_vector_type(4))) v, int __attribute__((ext_vector_type(4))) rsrc,
-                                   int voffset, int soffset, int aux) __asm("llvm.amdgcn.raw.buffer.store.v4f32");
-
 namespace {
 
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-typedef float float4v __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef int i32x4 __attribute__((ext_vector_type(4)));
-
-constexpr int TBN = 256;              // weight rows per tile
-constexpr int TWAVES = 8;             // 2 per SIMD
 constexpr int SB = 2;                 // blocks per stage
-constexpr int FRAG = 1024;            // bytes per activation fragment (16 tokens x 32 k, one limb)
 
 // Wave grid per token-tile height BM: WGM x WGN waves, each a (BM / WGM) x
 // (TBN / WGN) tile of 16 x 16 MFMA tiles.
@@ -81,15 +67,6 @@ template <>
 struct TFmt<WH_TYPE_Q8_0> {
   static constexpr int TS = 34, QOFF = 2;
 };
-// the repacked K-quant formats (f32 scale)
-template <>
-struct TFmt<wh::kGemmQ4F> {
-  static constexpr int TS = 20, QOFF = 4;
-};
-template <>
-struct TFmt<wh::kGemmQ8H> {
-  static constexpr int TS = 20, QOFF = 4;
-};
 // block value d q + m (Q4_1): the m of each block are collected, as the
 // stages stream past, into the B operand of products against the
 // activations' block sums, over windows of 32 blocks
@@ -97,17 +74,16 @@ template <int TYPE>
 constexpr bool has_min() { return TYPE == WH_TYPE_Q4_1; }
 // int8 quants in natural element order (else 4-bit quants in nibble order)
 template <int TYPE>
-constexpr bool q8_like() { return TYPE == WH_TYPE_Q8_0 || TYPE == wh::kGemmQ8H; }
-// f32 block scale (else f16)
-template <int TYPE>
-constexpr bool f32_scale() { return TYPE == wh::kGemmQ4F || TYPE == wh::kGemmQ8H; }
+constexpr bool q8_like() { return TYPE == WH_TYPE_Q8_0; }
+// K-quant stage records (gemm_sb.hpp): packed and sized here, multiplied there
+__host__ __device__ inline bool is_sb(int type) { return type == wh::kGemmQ4S || type == wh::kGemmQ6S; }
 // the packing writes the activations' sums over each unit of the minimum
-// term (Q4_1: 32-element block; kGemmQ4F: 256-element super-block) as two
+// term (Q4_1: 32-element block; kGemmQ4S: 256-element super-block) as two
 // fp16 limbs, rows of units rounded up to 8
-inline bool needs_bsum(int type) { return type == WH_TYPE_Q4_1 || type == wh::kGemmQ4F; }
+inline bool needs_bsum(int type) { return type == WH_TYPE_Q4_1 || type == wh::kGemmQ4S; }
 // units per token row in the sums' layout (4 bytes each: two fp16 limbs)
 inline size_t bsum_groups(int type, size_t k) {
-  return type == wh::kGemmQ4F ? wh::q4f_dmin_stride(k) : (k / 32 + 7) / 8 * 8;
+  return type == wh::kGemmQ4S ? wh::q4s_dmin_stride(k) : (k / 32 + 7) / 8 * 8;
 }
 // dwords per weight row per stage (SB whole blocks)
 template <int TYPE>
@@ -141,7 +117,8 @@ template <int TYPE, int BM>
 constexpr size_t tiled_lds_bytes() { return static_cast<size_t>(nstage<TYPE, BM>()) * stage_bytes<TYPE, BM>(); }
 
 // K-slot order of an MFMA operand: k-slot s (0..7) of k-group g (0..3) holds
-// block element 8g + s for the int8 formats, and for the 4-bit formats element
+// block element 8g + s for the int8 format, element 64 (b / 2) + 16 g + 8 (b %
+// 2) + s of the row for step b of the K-quant stage records, and for the 4-bit formats element
 // (s < 4 ? 0 : 16) + 4g + {0, 2, 1, 3}[s % 4], the order unpack_q4 below
 // produces the quants in.
 
@@ -149,7 +126,7 @@ constexpr size_t tiled_lds_bytes() { return static_cast<size_t>(nstage<TYPE, BM>
 // One workgroup per token row t of the padded tile grid (token tiles of bm
 // rows).  Rows t >= n_tokens are written as zeros.  rscale[t] = 2^e with
 // max|x_t| * 2^-e in [2^13, 2^14); bsum = the sums S of hi + lo over each
-// unit of the minimum term (Q4_1: 32-element block; kGemmQ4F: 256-element
+// unit of the minimum term (Q4_1: 32-element block; kGemmQ4S: 256-element
 // super-block) as the A operand of its products: fp16 limbs
 // hi = fp16(S 2^-10), lo = fp16(S 2^-10 - hi) (|S| < 2^22, so no overflow),
 // laid out [t][limb][units rounded up to 8], zero past the row's units.
@@ -163,8 +140,6 @@ constexpr size_t tiled_lds_bytes() { return static_cast<size_t>(nstage<TYPE, BM>
 // (tensor_utils.rs:446-480; kPackNorm); or the SwiGLU of two rows,
 // (g * (1 / (1 + exp(-g)))) * u with g = x, u = x2 (tensor_utils.rs:512-532;
 // kPackSwiglu).  The FFN's elementwise steps thereby never go through HBM.
-// Rows of x are kx long; k is the packed length: kx, or 2 kx for kGemmQ8H,
-// whose 32-element blocks hold 16 elements of x and 16 zeros.
 constexpr int PPT = 2;
 constexpr int kPackMaxThreads = 1024;
 constexpr int kPackPlain = 0, kPackNorm = 1, kPackSwiglu = 2;
@@ -172,7 +147,7 @@ constexpr int kPackPlain = 0, kPackNorm = 1, kPackSwiglu = 2;
 template <int MODE, bool XB = false>
 __global__ __launch_bounds__(kPackMaxThreads) void pack_a_kernel(const float* __restrict__ x, const float* __restrict__ x2,
                                                      const float* __restrict__ gamma, float eps, int n_tokens,
-                                                     int k, int kx, int type, int bm, _Float16* __restrict__ frag,
+                                                     int k, int type, int bm, _Float16* __restrict__ frag,
                                                      float* __restrict__ rscale, float* __restrict__ bsum,
                                                      uint32_t* __restrict__ sk_flags, int sk_n) {
   // the stream-K flags of the GEMMs that read this packing start cleared
@@ -183,14 +158,15 @@ __global__ __launch_bounds__(kPackMaxThreads) void pack_a_kernel(const float* __
   const int NTH = static_cast<int>(blockDim.x), nw = NTH >> 6;
   const int t = blockIdx.x;
   const bool live = t < n_tokens;
-  const float* xr = x + static_cast<size_t>(live ? t : 0) * kx;
-  const float* ur = MODE == kPackSwiglu ? x2 + static_cast<size_t>(live ? t : 0) * kx : nullptr;
+  const float* xr = x + static_cast<size_t>(live ? t : 0) * k;
+  const float* ur = MODE == kPackSwiglu ? x2 + static_cast<size_t>(live ? t : 0) * k : nullptr;
   const int nb = k / 32, npairs = nb * 4;
   const int nchunks = (npairs + NTH * PPT - 1) / (NTH * PPT);
-  const bool q8 = type == WH_TYPE_Q8_0 || type == wh::kGemmQ8H;
-  const bool pad = type == wh::kGemmQ8H;
-  // offset in the row of x of pair (b, g)'s first element, -1 for padding
-  auto elem_off = [&](int b, int g) { return pad ? (g < 2 ? 16 * b + 8 * g : -1) : 32 * b + (q8 ? 8 * g : 4 * g); };
+  const bool sb = is_sb(type), q8 = type == WH_TYPE_Q8_0 || sb;
+  // offset in the row of x of pair (b, g)'s first element
+  auto elem_off = [&](int b, int g) {
+    return sb ? 64 * (b >> 1) + 16 * g + 8 * (b & 1) : 32 * b + (q8 ? 8 * g : 4 * g);
+  };
   float4 va[PPT], vb[PPT];
   auto load = [&](int c) {
 #pragma unroll
@@ -201,8 +177,8 @@ __global__ __launch_bounds__(kPackMaxThreads) void pack_a_kernel(const float* __
       if (live && off >= 0) {
         const float* src = xr + off;
         if constexpr (XB) {
-          // row t of bf16 x: element e at byte 2 (t kx + e)
-          const uint16_t* xb = reinterpret_cast<const uint16_t*>(x) + static_cast<size_t>(t) * kx + off;
+          // row t of bf16 x: element e at byte 2 (t k + e)
+          const uint16_t* xb = reinterpret_cast<const uint16_t*>(x) + static_cast<size_t>(t) * k + off;
           auto widen = [](uint2 u) {
             return float4{__builtin_bit_cast(float, u.x << 16), __builtin_bit_cast(float, u.x & 0xFFFF0000u),
                           __builtin_bit_cast(float, u.y << 16), __builtin_bit_cast(float, u.y & 0xFFFF0000u)};
@@ -258,7 +234,7 @@ __global__ __launch_bounds__(kPackMaxThreads) void pack_a_kernel(const float* __
     __syncthreads();
     float tot = 0.f;
     for (int w = 0; w < nw; w++) tot += red2[w];
-    rms = sqrtf(tot / static_cast<float>(kx) + eps);
+    rms = sqrtf(tot / static_cast<float>(k) + eps);
   }
   float mx = 0.f;
   for (int c = 0; c < nchunks; c++) {
@@ -326,7 +302,7 @@ __global__ __launch_bounds__(kPackMaxThreads) void pack_a_kernel(const float* __
         // (p = 32 sb + ..; rows are whole super-blocks, so all 32 are live)
         part += __shfl_xor(part, 1, 64);
         part += __shfl_xor(part, 2, 64);
-        const bool sup = type == wh::kGemmQ4F;
+        const bool sup = sb;
         if (sup) {
           part += __shfl_xor(part, 4, 64);
           part += __shfl_xor(part, 8, 64);
@@ -358,7 +334,6 @@ __device__ __forceinline__ half8 unpack_q4(uint32_t u) {
   constexpr float OFF_LO = TYPE == WH_TYPE_Q4_0 ? -1032.f : -1024.f;
   constexpr float OFF_HI = TYPE == WH_TYPE_Q4_0 ? -72.f : -64.f;
   const uint32_t t8 = u >> 8;
-  typedef _Float16 half2v __attribute__((ext_vector_type(2)));
   const half2v lo_a = __builtin_bit_cast(half2v, (u & 0x000F000Fu) | 0x64006400u);
   const half2v lo_b = __builtin_bit_cast(half2v, (t8 & 0x000F000Fu) | 0x64006400u);
   const half2v hi_a = __builtin_bit_cast(half2v, (u & 0x00F000F0u) | 0x64006400u);
@@ -380,7 +355,6 @@ __device__ __forceinline__ half8 unpack_q4(uint32_t u) {
 // half of each 16-bit lane with v_perm, (b ^ 0x80) | 0x6400 = 1024 + q + 128,
 // minus 1152.
 __device__ __forceinline__ half8 unpack_q8(uint32_t u0, uint32_t u1) {
-  typedef _Float16 half2v __attribute__((ext_vector_type(2)));
   const half2v off = {static_cast<_Float16>(-1152.f), static_cast<_Float16>(-1152.f)};
   half8 out;
   const uint32_t w[2] = {u0, u1};
@@ -410,7 +384,6 @@ __device__ __forceinline__ uint32_t and_or(uint32_t u, uint32_t mask, uint32_t m
 // be computed at different points of the schedule.
 template <int TYPE>
 __device__ __forceinline__ void unpack_part(int p, uint32_t u0, uint32_t u1, uint32_t magic, half8& out) {
-  typedef _Float16 half2v __attribute__((ext_vector_type(2)));
   half2v r;
   if constexpr (q8_like<TYPE>()) {
     const half2v off = {static_cast<_Float16>(-1152.f), static_cast<_Float16>(-1152.f)};
@@ -434,72 +407,7 @@ __device__ __forceinline__ void unpack_part(int p, uint32_t u0, uint32_t u1, uin
   out[2 * p + 1] = r[1];
 }
 
-// Global -> LDS copies (global_load_lds): lane l's 16 (or 4) bytes at
-// base + voff land at LDS address lds + 16 l (4 l).  Issued through inline asm
-// so that the compiler does not treat them as pending LDS writes (it would
-// otherwise wait for every copy in flight before each LDS read); completion
-// is tracked explicitly with wait_vmcnt.  The copy reads its LDS address from
-// M0, a register the compiler reserves: the statement saves M0 in an SGPR of
-// its own, sets it (one wait state before the copy reads it, as GFX9-family
-// parts require after an SALU write of M0) and restores it, so M0 holds the
-// compiler's value again after every copy.
-__device__ __forceinline__ void copy16_to_lds(const void* base, uint32_t voff, uint32_t lds) {
-  const uint32_t m0 = __builtin_amdgcn_readfirstlane(lds);  // wave-uniform by construction
-  uint32_t saved;
-  asm volatile(
-      "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0"
-      : "=&s"(saved)
-      : "v"(voff), "s"(base), "s"(m0)
-      : "memory");
-}
-__device__ __forceinline__ void copy4_to_lds(const void* base, uint32_t voff, uint32_t lds) {
-  const uint32_t m0 = __builtin_amdgcn_readfirstlane(lds);
-  uint32_t saved;
-  asm volatile(
-      "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2\n\ts_mov_b32 m0, %0"
-      : "=&s"(saved)
-      : "v"(voff), "s"(base), "s"(m0)
-      : "memory");
-}
-__device__ __forceinline__ uint32_t lds_addr(const void* p) {
-  // generic -> LDS address space (an address-space cast), then its 32-bit address
-  return static_cast<uint32_t>((uintptr_t)((const __attribute__((address_space(3))) uint8_t*)p));
-}
-
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-  static_assert(N >= 0 && N < 64, "vmcnt range");
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-
-// Stream-K partial tiles: a buffer resource over one slot (128 KB or less)
-// and the cache policy of the slot's loads and stores, sc1 (bit 4 of the
-// buffer instructions' cache-policy operand on gfx950): the policy the memory
-// model gives agent-scope atomic loads and stores, coherent across the XCDs'
-// L2s without a cache-wide writeback or invalidate.
-constexpr int kSkCoherent = 16;
-__device__ __forceinline__ int __attribute__((ext_vector_type(4))) sk_rsrc(const float* base) {
-  const uint64_t a = reinterpret_cast<uint64_t>(base);
-  int __attribute__((ext_vector_type(4))) r;
-  r[0] = static_cast<int>(static_cast<uint32_t>(a));
-  r[1] = static_cast<int>(static_cast<uint32_t>(a >> 32) & 0xFFFFu);
-  r[2] = 1 << 20;  // 1 MB of records: every slot offset is in range
-  r[3] = 0x00020000;
-  return r;
-}
-
 // ---------------------------------------------------------------- GEMM
-// Waits until at most min(n, J) stages of N copies each are in flight.
-template <int N, int J>
-__device__ __forceinline__ void wait_stages(int n) {
-  if constexpr (J == 0) {
-    wait_vmcnt<0>();
-  } else {
-    if (n >= J) wait_vmcnt<J * N>();
-    else wait_stages<N, J - 1>(n);
-  }
-}
-
 // Y (or split-K partial plane blockIdx.y) for one BM x 256 tile over blocks
 // [kb0, kb1).  Grid: x = tiles (XCD-grouped order), y = K splits.
 // SK (stream-K; one workgroup per CU, used when the tiles do not fill the CUs
@@ -526,7 +434,7 @@ __device__ __forceinline__ void wait_stages(int n) {
 template <int TYPE, int BM, bool FFNP = false, bool SK = false, bool LO = true>
 __global__ __launch_bounds__(TWAVES * 64, 1) void gemm_tiled_kernel(
     const uint8_t* __restrict__ W, const uint8_t* __restrict__ W2, const _Float16* __restrict__ frag,
-    const float* __restrict__ rscale, const float* __restrict__ bsum, const float* __restrict__ dmin,
+    const float* __restrict__ rscale, const float* __restrict__ bsum,
     float* __restrict__ y, int n_tokens, int n_rows, int nb, int blocks_per_split, int tiles_n, int n_tiles,
     uint32_t* __restrict__ sk_flags, float* __restrict__ sk_part, int sk_upw, int sk_sub, uint32_t sk_wait) {
   using C = TCfg<BM>;
@@ -742,12 +650,7 @@ __global__ __launch_bounds__(TWAVES * 64, 1) void gemm_tiled_kernel(
         const int row = FFNP ? ((n & 1) ? HALF : 0) + wn / 2 + 16 * (n >> 1) + ln : wn + 16 * n + ln;
         const uint8_t* rb = bslot + row * (DWB * 4) + j * TS;     // this block's bytes
         const uint16_t* r16 = reinterpret_cast<const uint16_t*>(rb);
-        if constexpr (TYPE == wh::kGemmQ8H) {
-          // 16 quants: k-groups 0, 1; groups 2, 3 are the zero padding
-          const uint32_t* q32 = reinterpret_cast<const uint32_t*>(rb + QOFF + 8 * (g & 1));
-          wq0[j][n] = g < 2 ? q32[0] : 0u;
-          wq1[j][n] = g < 2 ? q32[1] : 0u;
-        } else if constexpr (TYPE == WH_TYPE_Q8_0) {
+        if constexpr (TYPE == WH_TYPE_Q8_0) {
           const uint16_t* q16 = reinterpret_cast<const uint16_t*>(rb + QOFF + 8 * g);
           wq0[j][n] = static_cast<uint32_t>(q16[0]) | (static_cast<uint32_t>(q16[1]) << 16);
           wq1[j][n] = static_cast<uint32_t>(q16[2]) | (static_cast<uint32_t>(q16[3]) << 16);
@@ -756,12 +659,8 @@ __global__ __launch_bounds__(TWAVES * 64, 1) void gemm_tiled_kernel(
           wq0[j][n] = static_cast<uint32_t>(q16[0]) | (static_cast<uint32_t>(q16[1]) << 16);
           wq1[j][n] = 0u;
         }
-        if constexpr (f32_scale<TYPE>()) {
-          wdm[j][n] = reinterpret_cast<const uint32_t*>(rb)[0];
-        } else {
-          wdm[j][n] = TYPE == WH_TYPE_Q4_1 ? (static_cast<uint32_t>(r16[0]) | (static_cast<uint32_t>(r16[1]) << 16))
-                                           : static_cast<uint32_t>(r16[0]);
-        }
+        wdm[j][n] = TYPE == WH_TYPE_Q4_1 ? (static_cast<uint32_t>(r16[0]) | (static_cast<uint32_t>(r16[1]) << 16))
+                                         : static_cast<uint32_t>(r16[0]);
       }
     }
     half8 bw[2];
@@ -808,11 +707,7 @@ __global__ __launch_bounds__(TWAVES * 64, 1) void gemm_tiled_kernel(
         // this pair becomes the pending one
 #pragma unroll
         for (int h = 0; h < 2; h++) {
-          if constexpr (f32_scale<TYPE>()) {
-            pd[h] = __uint_as_float(wdm[j][2 * np + h]);
-          } else {
-            pd[h] = whd::f16_bits_to_f32(wdm[j][2 * np + h] & 0xFFFFu);
-          }
+          pd[h] = whd::f16_bits_to_f32(wdm[j][2 * np + h] & 0xFFFFu);
           asm("" : "+v"(pd[h]));  // in a VGPR: the FMAs are then plain v_fmac_f32
         }
         bw[0] = bn[0];
@@ -899,69 +794,6 @@ __global__ __launch_bounds__(TWAVES * 64, 1) void gemm_tiled_kernel(
     }
   }
 
-  if constexpr (TYPE == wh::kGemmQ4F) {
-    // Q4_K's dmin: acc += dmin[row][sb] * S[token][sb] over this split's
-    // super-blocks (split bounds are multiples of 8 blocks), S the packing's
-    // super-block sums in the same scaled domain as acc.  Under stream-K the
-    // workgroup that finishes a tile adds the term of every super-block (the
-    // other owners' parts carry none).  As matrix-core products over windows
-    // of 32 super-blocks: lane group g holds super-blocks 8g .. 8g + 7 of the
-    // window in both operands (B: the fp16 dmin table, those outside
-    // [sb_lo, sb_hi) masked to zero; A: S as hi + lo fp16 limbs of S 2^-10),
-    // and one fma per output adds 2^10 times the window's sum.
-    static_assert(!FFNP, "the gate / up pass has no dmin term");
-    const int nsb = nb / 8, nsbp = (nsb + 7) & ~7;
-    const int sb_lo = SK ? 0 : st_a * SB / 8, sb_hi = SK ? nsb : st_b * SB / 8;
-    const uint16_t* dm16 = reinterpret_cast<const uint16_t*>(dmin);
-    const uint16_t* s16 = reinterpret_cast<const uint16_t*>(bsum);
-    // the lane index opaque here, so that the loads' offsets are formed here
-    // and not held in registers through the stage loop; 32-bit offsets (both
-    // arrays hold fewer than 2^28 halves: the launcher keeps the weight and
-    // fragment bytes below 2^32)
-    int lnv = ln;
-    asm volatile("" : "+v"(lnv));
-    for (int w0 = sb_lo & ~31; w0 < sb_hi; w0 += 32) {
-      const int s0 = w0 + 8 * g;                  // this lane's first super-block
-      const bool in = s0 < nsbp;                  // inside the table's rows
-      uint32_t mk[4];
-#pragma unroll
-      for (int d = 0; d < 4; d++) {
-        const int a = s0 + 2 * d;
-        mk[d] = (a >= sb_lo && a < sb_hi ? 0x0000FFFFu : 0u) | (a + 1 >= sb_lo && a + 1 < sb_hi ? 0xFFFF0000u : 0u);
-      }
-      u32x4 bd[NT];
-#pragma unroll
-      for (int n = 0; n < NT; n++) {
-        const uint32_t off = static_cast<uint32_t>(min(r0 + wn + 16 * n + lnv, n_rows - 1) * nsbp + s0);
-        bd[n] = in ? *reinterpret_cast<const u32x4*>(dm16 + off) : u32x4{0u, 0u, 0u, 0u};
-      }
-      u32x4 sh[IT], sl[IT];
-#pragma unroll
-      for (int i = 0; i < IT; i++) {
-        const uint32_t off = static_cast<uint32_t>((t0 + wm + 16 * i + lnv) * 2 * nsbp + s0);
-        sh[i] = in ? *reinterpret_cast<const u32x4*>(s16 + off) : u32x4{0u, 0u, 0u, 0u};
-        sl[i] = in ? *reinterpret_cast<const u32x4*>(s16 + off + nsbp) : u32x4{0u, 0u, 0u, 0u};
-      }
-      __builtin_amdgcn_sched_barrier(0);  // every load issued before the first use
-#pragma unroll
-      for (int n = 0; n < NT; n++)
-#pragma unroll
-        for (int d = 0; d < 4; d++) bd[n][d] &= mk[d];
-#pragma unroll
-      for (int i = 0; i < IT; i++) {
-#pragma unroll
-        for (int n = 0; n < NT; n++) {
-          float4v t = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, sh[i]), __builtin_bit_cast(half8, bd[n]),
-                                                             float4v{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-          t = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, sl[i]), __builtin_bit_cast(half8, bd[n]), t, 0, 0, 0);
-#pragma unroll
-          for (int r = 0; r < 4; r++) acc[i][n][r] = __builtin_fmaf(1024.f, t[r], acc[i][n][r]);
-        }
-        __builtin_amdgcn_sched_barrier(0);  // one token group's products at a time
-      }
-    }
-  }
-
   if constexpr (FFNP) {
     // h = silu(g) * u for the gate / up pairs, as (g * (1 / (1 + e^-g))) * u
 #pragma unroll
@@ -1013,19 +845,21 @@ __global__ __launch_bounds__(256) void tiled_splitk_reduce_kernel(const float* _
 
 // Token-tile height for a token count: the smallest of 16, 32, 64, 128 that
 // holds it (one tile) or 128 beyond.
-int tile_bm(size_t n_tokens) { return n_tokens <= 16 ? 16 : (n_tokens <= 32 ? 32 : (n_tokens <= 64 ? 64 : 128)); }
+int tile_bm(int type, size_t n_tokens) {
+  if (n_tokens <= 16 && !is_sb(type)) return 16;  // (the K-quant kernel starts at 32)
+  return n_tokens <= 32 ? 32 : (n_tokens <= 64 ? 64 : 128);
+}
 
 // Stream-K grid for n_tiles tiles of tile_st stages each: one workgroup per
 // CU whenever the tiles do not fill the CUs evenly (a last round with idle
 // CUs, or fewer tiles than CUs, where split-K planes and a reduce would
 // otherwise be needed) and every workgroup's share is at least 8 stages; 0
 // (one workgroup per tile) otherwise.  Every block format of the kernel.
+// (The K-quant kernel's units are super-blocks of four stages.)
 int sk_grid(int type, size_t n_tiles, size_t tile_st) {
-  if (type != WH_TYPE_Q4_0 && type != WH_TYPE_Q4_1 && type != WH_TYPE_Q8_0 && type != wh::kGemmQ4F &&
-      type != wh::kGemmQ8H)
-    return 0;
   const size_t g = static_cast<size_t>(wh::cu_count());
   if (g == 0 || g % 8 != 0 || n_tiles % g == 0) return 0;
+  if (is_sb(type)) return (n_tiles * (tile_st / 4) + g - 1) / g >= 2 ? static_cast<int>(g) : 0;
   const size_t upw = (n_tiles * tile_st + g - 1) / g;
   return upw >= 8 ? static_cast<int>(g) : 0;
 }
@@ -1044,7 +878,7 @@ std::atomic<uint32_t> g_sk_wait{100000u};
 
 template <int TYPE, int BM, bool LO>
 int launch_bm_lo(const uint8_t* w, size_t n_rows, size_t k, size_t n_tokens, const _Float16* frag,
-              const float* rs, const float* bs, const float* dmin, float* part, int splits, const SkWs& sk,
+              const float* rs, const float* bs, float* part, int splits, const SkWs& sk,
               hipStream_t s) {
   const int nb = static_cast<int>(k / 32);
   const int tiles_n = static_cast<int>((n_rows + TBN - 1) / TBN);
@@ -1056,18 +890,17 @@ int launch_bm_lo(const uint8_t* w, size_t n_rows, size_t k, size_t n_tokens, con
       const int upw = (n_tiles * (nb / SB) + sk.g - 1) / sk.g;
       WH_ENSURE_LDS(lds, &gemm_tiled_kernel<TYPE, BM, false, true, LO>);
       gemm_tiled_kernel<TYPE, BM, false, true, LO><<<static_cast<unsigned>(sk.g), TWAVES * 64, lds, s>>>(
-          w, nullptr, frag, rs, bs, dmin, part, static_cast<int>(n_tokens), static_cast<int>(n_rows), nb, nb, tiles_n,
+          w, nullptr, frag, rs, bs, part, static_cast<int>(n_tokens), static_cast<int>(n_rows), nb, nb, tiles_n,
           n_tiles, sk.flags, sk.part, upw, sk.sub, g_sk_wait.load(std::memory_order_relaxed));
       WH_LAUNCH_CHECK("tiled gemm kernel launch");
       return WH_OK;
     }
   }
   int bps = (nb + splits - 1) / splits;
-  constexpr int ALIGN = TYPE == wh::kGemmQ4F ? 8 : SB;   // kGemmQ4F: whole super-blocks per split
-  bps = (bps + ALIGN - 1) / ALIGN * ALIGN;
+  bps = (bps + SB - 1) / SB * SB;
   WH_ENSURE_LDS(lds, &gemm_tiled_kernel<TYPE, BM, false, false, LO>);
   dim3 grid(static_cast<unsigned>(n_tiles), static_cast<unsigned>(splits));
-  gemm_tiled_kernel<TYPE, BM, false, false, LO><<<grid, TWAVES * 64, lds, s>>>(w, nullptr, frag, rs, bs, dmin, part,
+  gemm_tiled_kernel<TYPE, BM, false, false, LO><<<grid, TWAVES * 64, lds, s>>>(w, nullptr, frag, rs, bs, part,
                                                            static_cast<int>(n_tokens), static_cast<int>(n_rows), nb,
                                                            bps, tiles_n, n_tiles, nullptr, nullptr, 0, 0, 0u);
   WH_LAUNCH_CHECK("tiled gemm kernel launch");
@@ -1079,12 +912,12 @@ int launch_bm_lo(const uint8_t* w, size_t n_rows, size_t k, size_t n_tokens, con
 // 128-token tiles of the 32-element block formats, the bf16 path's shapes).
 template <int TYPE, int BM>
 int launch_bm(const uint8_t* w, size_t n_rows, size_t k, size_t n_tokens, const _Float16* frag,
-              const float* rs, const float* bs, const float* dmin, float* part, int splits, const SkWs& sk,
+              const float* rs, const float* bs, float* part, int splits, const SkWs& sk,
               hipStream_t s, bool lo) {
   if constexpr ((TYPE == WH_TYPE_Q4_0 || TYPE == WH_TYPE_Q4_1 || TYPE == WH_TYPE_Q8_0) && BM >= 32) {
-    if (!lo) return launch_bm_lo<TYPE, BM, false>(w, n_rows, k, n_tokens, frag, rs, bs, dmin, part, splits, sk, s);
+    if (!lo) return launch_bm_lo<TYPE, BM, false>(w, n_rows, k, n_tokens, frag, rs, bs, part, splits, sk, s);
   }
-  return launch_bm_lo<TYPE, BM, true>(w, n_rows, k, n_tokens, frag, rs, bs, dmin, part, splits, sk, s);
+  return launch_bm_lo<TYPE, BM, true>(w, n_rows, k, n_tokens, frag, rs, bs, part, splits, sk, s);
 }
 
 // The FFN's gate and up (n_ff rows each) in one pass: h = silu(gate x) * (up x).
@@ -1100,14 +933,14 @@ int launch_ffn_bm(const uint8_t* gate, const uint8_t* up, size_t n_ff, size_t k,
     const int upw = (n_tiles * (nb / SB) + sk.g - 1) / sk.g;
     WH_ENSURE_LDS(lds, &gemm_tiled_kernel<TYPE, BM, true, true>);
     gemm_tiled_kernel<TYPE, BM, true, true><<<static_cast<unsigned>(sk.g), TWAVES * 64, lds, s>>>(
-        gate, up, frag, rs, bs, nullptr, h, static_cast<int>(n_tokens), static_cast<int>(n_ff), nb, nb, tiles_n,
+        gate, up, frag, rs, bs, h, static_cast<int>(n_tokens), static_cast<int>(n_ff), nb, nb, tiles_n,
         n_tiles, sk.flags, sk.part, upw, sk.sub, g_sk_wait.load(std::memory_order_relaxed));
     WH_LAUNCH_CHECK("tiled ffn gate/up kernel launch");
     return WH_OK;
   }
   WH_ENSURE_LDS(lds, &gemm_tiled_kernel<TYPE, BM, true>);
   gemm_tiled_kernel<TYPE, BM, true><<<static_cast<unsigned>(n_tiles), TWAVES * 64, lds, s>>>(
-      gate, up, frag, rs, bs, nullptr, h, static_cast<int>(n_tokens), static_cast<int>(n_ff), nb, nb, tiles_n,
+      gate, up, frag, rs, bs, h, static_cast<int>(n_tokens), static_cast<int>(n_ff), nb, nb, tiles_n,
       n_tiles, nullptr, nullptr, 0, 0, 0u);
   WH_LAUNCH_CHECK("tiled ffn gate/up kernel launch");
   return WH_OK;
@@ -1116,7 +949,7 @@ int launch_ffn_bm(const uint8_t* gate, const uint8_t* up, size_t n_ff, size_t k,
 template <int TYPE>
 int launch_ffn_typed(const uint8_t* gate, const uint8_t* up, size_t n_ff, size_t k, size_t n_tokens,
                      const _Float16* frag, const float* rs, const float* bs, float* h, const SkWs& sk, hipStream_t s) {
-  switch (tile_bm(n_tokens)) {
+  switch (tile_bm(TYPE, n_tokens)) {
     case 16: return launch_ffn_bm<TYPE, 16>(gate, up, n_ff, k, n_tokens, frag, rs, bs, h, sk, s);
     case 32: return launch_ffn_bm<TYPE, 32>(gate, up, n_ff, k, n_tokens, frag, rs, bs, h, sk, s);
     case 64: return launch_ffn_bm<TYPE, 64>(gate, up, n_ff, k, n_tokens, frag, rs, bs, h, sk, s);
@@ -1126,13 +959,13 @@ int launch_ffn_typed(const uint8_t* gate, const uint8_t* up, size_t n_ff, size_t
 
 template <int TYPE>
 int launch_typed(const uint8_t* w, size_t n_rows, size_t k, size_t n_tokens, const _Float16* frag,
-                 const float* rs, const float* bs, const float* dmin, float* part, int splits, const SkWs& sk,
+                 const float* rs, const float* bs, float* part, int splits, const SkWs& sk,
                  hipStream_t s, bool lo) {
-  switch (tile_bm(n_tokens)) {
-    case 16: return launch_bm<TYPE, 16>(w, n_rows, k, n_tokens, frag, rs, bs, dmin, part, splits, sk, s, lo);
-    case 32: return launch_bm<TYPE, 32>(w, n_rows, k, n_tokens, frag, rs, bs, dmin, part, splits, sk, s, lo);
-    case 64: return launch_bm<TYPE, 64>(w, n_rows, k, n_tokens, frag, rs, bs, dmin, part, splits, sk, s, lo);
-    default: return launch_bm<TYPE, 128>(w, n_rows, k, n_tokens, frag, rs, bs, dmin, part, splits, sk, s, lo);
+  switch (tile_bm(TYPE, n_tokens)) {
+    case 16: return launch_bm<TYPE, 16>(w, n_rows, k, n_tokens, frag, rs, bs, part, splits, sk, s, lo);
+    case 32: return launch_bm<TYPE, 32>(w, n_rows, k, n_tokens, frag, rs, bs, part, splits, sk, s, lo);
+    case 64: return launch_bm<TYPE, 64>(w, n_rows, k, n_tokens, frag, rs, bs, part, splits, sk, s, lo);
+    default: return launch_bm<TYPE, 128>(w, n_rows, k, n_tokens, frag, rs, bs, part, splits, sk, s, lo);
   }
 }
 
@@ -1162,8 +995,8 @@ static size_t tiled_ts(int type) {
     case WH_TYPE_Q4_0: return TFmt<WH_TYPE_Q4_0>::TS;
     case WH_TYPE_Q4_1: return TFmt<WH_TYPE_Q4_1>::TS;
     case WH_TYPE_Q8_0: return TFmt<WH_TYPE_Q8_0>::TS;
-    case kGemmQ4F: return TFmt<kGemmQ4F>::TS;
-    case kGemmQ8H: return TFmt<kGemmQ8H>::TS;
+    case kGemmQ4S: return 20;  // half of a 64-element stage record
+    case kGemmQ6S: return 40;
     default: return 0;
   }
 }
@@ -1171,7 +1004,7 @@ static size_t tiled_ts(int type) {
 bool gemm_tiled_ok(int type, const void* w, const float* x, size_t n_rows, size_t k, size_t n_tokens) {
   const size_t ts = tiled_ts(type);
   if (ts == 0 || k == 0 || k % (32 * SB) != 0 || !aligned(w, 4) || !aligned(x, 16) || ((k / 32) * ts) % 4 != 0) return false;
-  const size_t bm = static_cast<size_t>(tile_bm(n_tokens));
+  const size_t bm = static_cast<size_t>(tile_bm(type, n_tokens));
   const size_t tm = (n_tokens + bm - 1) / bm * bm;
   const size_t lim = static_cast<size_t>(1) << 32;
   if (n_rows * (k / 32) * ts >= lim || tm * k * 4 >= lim) return false;
@@ -1181,20 +1014,24 @@ bool gemm_tiled_ok(int type, const void* w, const float* x, size_t n_rows, size_
     case WH_TYPE_Q4_0: lds = lds_typed<WH_TYPE_Q4_0>(b); break;
     case WH_TYPE_Q4_1: lds = lds_typed<WH_TYPE_Q4_1>(b); break;
     case WH_TYPE_Q8_0: lds = lds_typed<WH_TYPE_Q8_0>(b); break;
-    case kGemmQ4F: lds = lds_typed<kGemmQ4F>(b); break;
-    default: lds = lds_typed<kGemmQ8H>(b); break;
+    default: lds = static_cast<size_t>(160) * 1024; break;  // gemm_sb.hpp: a ring in all of the LDS
   }
   return lds <= max_lds_per_block();
 }
 
 // Split-K factor: the largest power of two up to 8 that keeps the workgroups
-// within one per CU and every split at least 16 blocks deep.
-int gemm_tiled_splits(size_t n_rows, size_t n_tokens, size_t k) {
-  const size_t bm = static_cast<size_t>(tile_bm(n_tokens));
+// within one per CU and every split at least 16 blocks deep (the K-quant
+// kernel: 16, and one super-block).
+int gemm_tiled_splits(int type, size_t n_rows, size_t n_tokens, size_t k) {
+  const size_t bm = static_cast<size_t>(tile_bm(type, n_tokens));
   const size_t tiles = ((n_rows + TBN - 1) / TBN) * ((n_tokens + bm - 1) / bm);
   const size_t nb = k / 32;
   const size_t cus = static_cast<size_t>(cu_count());
   int s = 1;
+  if (is_sb(type)) {  // whole super-blocks, down to one per split
+    while (s < 16 && tiles * s * 2 <= cus && k / 256 >= static_cast<size_t>(2 * s)) s *= 2;
+    return s;
+  }
   while (s < 8 && tiles * s * 2 <= cus && nb / (2 * s) >= 16) s *= 2;
   return s;
 }
@@ -1205,43 +1042,39 @@ int gemm_tiled_splits(size_t n_rows, size_t n_tokens, size_t k) {
 // Token tiles of 16 and 32 keep split-K: their stages are short, and the
 // hand-off of a partial tile costs more than the reduce it replaces (M=32,
 // 14336 x 4096: 31.9 against 31.3 us).
-// The K-quant formats keep split-K too (their FFN at M=512: 462 against 442
-// us with stream-K in the down projection); their tiles take stream-K only
-// where they would leave CUs idle in a last round.
 static int sk_plain(int type, size_t n_rows, size_t n_tokens, size_t k) {
-  const size_t bm = static_cast<size_t>(tile_bm(n_tokens));
+  const size_t bm = static_cast<size_t>(tile_bm(type, n_tokens));
   if (bm < 64) return 0;
-  if ((type == kGemmQ4F || type == kGemmQ8H) && gemm_tiled_splits(n_rows, n_tokens, k) > 1) return 0;
   return sk_grid(type, ((n_tokens + bm - 1) / bm) * ((n_rows + TBN - 1) / TBN), k / 32 / SB);
 }
 // Split-K factor of the GEMM over n_rows rows: 1 where it runs stream-K.
 static int tiled_splits(int type, size_t n_rows, size_t n_tokens, size_t k) {
-  return sk_plain(type, n_rows, n_tokens, k) ? 1 : gemm_tiled_splits(n_rows, n_tokens, k);
+  return sk_plain(type, n_rows, n_tokens, k) ? 1 : gemm_tiled_splits(type, n_rows, n_tokens, k);
 }
 static int sk_slots(int type, size_t n_rows, size_t n_tokens, size_t k) {
   const int g = sk_plain(type, n_rows, n_tokens, k);
   if (g) return g;
-  if (gemm_tiled_splits(2 * n_rows, n_tokens, k) == 1 && tile_bm(n_tokens) >= 64) {
-    const size_t bm = static_cast<size_t>(tile_bm(n_tokens));
+  if (gemm_tiled_splits(type, 2 * n_rows, n_tokens, k) == 1 && tile_bm(type, n_tokens) >= 64) {
+    const size_t bm = static_cast<size_t>(tile_bm(type, n_tokens));
     return sk_grid(type, ((n_tokens + bm - 1) / bm) * ((n_rows + TBN / 2 - 1) / (TBN / 2)), k / 32 / SB);
   }
   return 0;
 }
 
-static size_t sk_bytes(int slots, size_t n_tokens) {
+static size_t sk_bytes(int type, int slots, size_t n_tokens) {
   return slots ? al256(static_cast<size_t>(slots) * 4) +
-                     static_cast<size_t>(slots) * static_cast<size_t>(tile_bm(n_tokens)) * TBN * 4
+                     static_cast<size_t>(slots) * static_cast<size_t>(tile_bm(type, n_tokens)) * TBN * 4
                : 0;
 }
 
 size_t gemm_tiled_workspace_bytes(int type, size_t n_rows, size_t n_tokens, size_t k) {
-  const size_t bm = static_cast<size_t>(tile_bm(n_tokens));
+  const size_t bm = static_cast<size_t>(tile_bm(type, n_tokens));
   const size_t tm = (n_tokens + bm - 1) / bm * bm;   // padded tokens
   size_t b = al256(tm * k * 4) + al256(tm * 4);
   if (needs_bsum(type)) b += al256(tm * bsum_groups(type, k) * 4);
   const int splits = tiled_splits(type, n_rows, n_tokens, k);
   if (splits > 1) b += al256(static_cast<size_t>(splits) * n_rows * n_tokens * 4);
-  return b + sk_bytes(sk_slots(type, n_rows, n_tokens, k), n_tokens);
+  return b + sk_bytes(type, sk_slots(type, n_rows, n_tokens, k), n_tokens);
 }
 
 // Workspace of one tiled GEMM: packed activations, row scales, Q4_1 block
@@ -1260,7 +1093,7 @@ struct TiledWs {
 
 static TiledWs tiled_ws(int type, size_t n_rows, size_t k, size_t n_tokens, void* workspace) {
   TiledWs t{};
-  t.bm = tile_bm(n_tokens);
+  t.bm = tile_bm(type, n_tokens);
   t.tm = (n_tokens + t.bm - 1) / t.bm * t.bm;
   char* ws = static_cast<char*>(workspace);
   t.frag = reinterpret_cast<_Float16*>(ws);
@@ -1284,33 +1117,63 @@ static TiledWs tiled_ws(int type, size_t n_rows, size_t k, size_t n_tokens, void
 
 template <int MODE, bool XB = false>
 static int tiled_pack(int type, const TiledWs& t, const float* x, const float* x2, const float* gamma, float eps,
-                      size_t n_tokens, size_t k, size_t kx, hipStream_t s) {
+                      size_t n_tokens, size_t k, hipStream_t s) {
   // threads per row: enough for PPT pairs each, 256 .. 1024
   const size_t npairs = k / 8;
   size_t threads = (npairs + PPT - 1) / PPT;
   threads = threads < 256 ? 256 : (threads > kPackMaxThreads ? kPackMaxThreads : (threads + 63) / 64 * 64);
   pack_a_kernel<MODE, XB><<<static_cast<unsigned>(t.tm), static_cast<unsigned>(threads), 0, s>>>(x, x2, gamma, eps, static_cast<int>(n_tokens),
-                                                                  static_cast<int>(k), static_cast<int>(kx), type, t.bm,
+                                                                  static_cast<int>(k), type, t.bm,
                                                                   t.frag, t.rs, t.bs, t.sk_flags, t.sk_n);
   WH_LAUNCH_CHECK("pack kernel launch");
   return WH_OK;
+}
+
+// The K-quant kernel over packed activations: y (or split-K planes) = W X, or
+// with w2 the FFN's gate and up in one pass.
+static int sb_run(int type, const uint8_t* w, const uint8_t* w2, size_t n_rows, size_t k, size_t n_tokens,
+                  const TiledWs& t, float* y, int splits, int sub, bool lo, hipStream_t s) {
+  SbGemm a{};
+  a.w = w;
+  a.w2 = w2;
+  a.frag = t.frag;
+  a.rs = t.rs;
+  a.bs = t.bs;
+  a.y = y;
+  a.n_tokens = static_cast<int>(n_tokens);
+  a.n_rows = static_cast<int>(n_rows);
+  a.k = static_cast<int>(k);
+  a.bm = t.bm;
+  a.splits = splits;
+  a.ffn = w2 != nullptr;
+  a.lo = lo;
+  const size_t tn = w2 ? TBN / 2 : TBN;
+  const size_t tiles = (n_rows + tn - 1) / tn * (t.tm / t.bm);
+  if (splits == 1 && t.sk_n > 0 && sk_grid(type, tiles, k / 64) == t.sk_n) {
+    a.sk_flags = t.sk_flags;
+    a.sk_part = t.sk_part;
+    a.sk_g = t.sk_n;
+    a.sk_sub = sub;
+    a.sk_wait = g_sk_wait.load(std::memory_order_relaxed);
+  }
+  return type == kGemmQ4S ? launch_gemm_sb_q4(a, s) : launch_gemm_sb_q6(a, s);
 }
 
 // The GEMM over packed activations (and the split-K reduce) into y.
 // sub: which of the GEMMs that read one packing this is (0, 1), so that their
 // stream-K flags differ.
 static int tiled_run(int type, const void* w, size_t n_rows, size_t k, size_t n_tokens, const TiledWs& t, float* y,
-                     hipStream_t s, const float* dmin = nullptr, int sub = 0, bool lo = true) {
+                     hipStream_t s, int sub = 0, bool lo = true) {
   const uint8_t* wp = static_cast<const uint8_t*>(w);
   float* part = t.splits > 1 ? t.part : y;
   const SkWs sk{t.sk_flags, t.sk_part, t.sk_n, sub};
   int st;
   switch (type) {
-    case WH_TYPE_Q4_0: st = launch_typed<WH_TYPE_Q4_0>(wp, n_rows, k, n_tokens, t.frag, t.rs, t.bs, dmin, part, t.splits, sk, s, lo); break;
-    case WH_TYPE_Q4_1: st = launch_typed<WH_TYPE_Q4_1>(wp, n_rows, k, n_tokens, t.frag, t.rs, t.bs, dmin, part, t.splits, sk, s, lo); break;
-    case WH_TYPE_Q8_0: st = launch_typed<WH_TYPE_Q8_0>(wp, n_rows, k, n_tokens, t.frag, t.rs, t.bs, dmin, part, t.splits, sk, s, lo); break;
-    case kGemmQ4F: st = launch_typed<kGemmQ4F>(wp, n_rows, k, n_tokens, t.frag, t.rs, t.bs, dmin, part, t.splits, sk, s, lo); break;
-    case kGemmQ8H: st = launch_typed<kGemmQ8H>(wp, n_rows, k, n_tokens, t.frag, t.rs, t.bs, dmin, part, t.splits, sk, s, lo); break;
+    case WH_TYPE_Q4_0: st = launch_typed<WH_TYPE_Q4_0>(wp, n_rows, k, n_tokens, t.frag, t.rs, t.bs, part, t.splits, sk, s, lo); break;
+    case WH_TYPE_Q4_1: st = launch_typed<WH_TYPE_Q4_1>(wp, n_rows, k, n_tokens, t.frag, t.rs, t.bs, part, t.splits, sk, s, lo); break;
+    case WH_TYPE_Q8_0: st = launch_typed<WH_TYPE_Q8_0>(wp, n_rows, k, n_tokens, t.frag, t.rs, t.bs, part, t.splits, sk, s, lo); break;
+    case kGemmQ4S:
+    case kGemmQ6S: st = sb_run(type, wp, nullptr, n_rows, k, n_tokens, t, part, t.splits, sub, lo, s); break;
     default: return set_error(WH_ERR_UNSUPPORTED_TYPE, "gemm: unsupported type %d", type);
   }
   if (st != WH_OK) return st;
@@ -1328,7 +1191,7 @@ static int tiled_run(int type, const void* w, size_t n_rows, size_t k, size_t n_
 int launch_gemm_tiled(int type, const void* w, size_t n_rows, size_t k, const float* x, size_t n_tokens,
                       float* y, void* workspace, hipStream_t s) {
   const TiledWs t = tiled_ws(type, n_rows, k, n_tokens, workspace);
-  int st = tiled_pack<kPackPlain>(type, t, x, nullptr, nullptr, 0.f, n_tokens, k, k, s);
+  int st = tiled_pack<kPackPlain>(type, t, x, nullptr, nullptr, 0.f, n_tokens, k, s);
   if (st) return st;
   return tiled_run(type, w, n_rows, k, n_tokens, t, y, s);
 }
@@ -1337,58 +1200,56 @@ int launch_gemm_tiled_bf16(int type, const void* w, size_t n_rows, size_t k, con
                            float* y, void* workspace, hipStream_t s) {
   const TiledWs t = tiled_ws(type, n_rows, k, n_tokens, workspace);
   int st = tiled_pack<kPackPlain, true>(type, t, reinterpret_cast<const float*>(x), nullptr, nullptr, 0.f, n_tokens,
-                                        k, k, s);
+                                        k, s);
   if (st) return st;
-  return tiled_run(type, w, n_rows, k, n_tokens, t, y, s, nullptr, 0, /*lo=*/false);
+  return tiled_run(type, w, n_rows, k, n_tokens, t, y, s, 0, /*lo=*/false);
 }
 
 // ------------------------------------------------------------- K-quants
 // The matrix is repacked (kquant.hip) into the front of the workspace, in the
-// GEMM format of kquant_gemm_type with reduction length kquant_gemm_k; the
-// packed activations and the rest of the GEMM's workspace follow it.
+// stage records of kquant_gemm_type; the packed activations and the rest of
+// the GEMM's workspace follow it.
 bool gemm_kquant_ok(int type, const void* w, const float* x, size_t n_rows, size_t k, size_t n_tokens) {
   if (!is_kquant(type) || k % 256 != 0 || !aligned(w, 16)) return false;
   // the repacked matrix is 256-byte aligned; any such address stands for it
   const void* repacked = reinterpret_cast<const void*>(static_cast<uintptr_t>(256));
-  return gemm_tiled_ok(kquant_gemm_type(type), repacked, x, n_rows, kquant_gemm_k(type, k), n_tokens);
-}
-
-// GEMM on a repacked K-quant matrix rp (its GEMM format, rows of k elements)
-// over packed activations t; Q4_K's dmin table follows the blocks.
-static int kquant_run(int type, const char* rp, size_t n_rows, size_t k, size_t n_tokens, const TiledWs& t,
-                      float* y, hipStream_t s, int sub = 0) {
-  // (the fp16 table, passed through the kernels' dmin pointer)
-  const float* dmin_t =
-      type == WH_TYPE_Q4_K ? reinterpret_cast<const float*>(rp + n_rows * (k / 32) * 20) : nullptr;
-  return tiled_run(kquant_gemm_type(type), rp, n_rows, kquant_gemm_k(type, k), n_tokens, t, y, s, dmin_t, sub);
+  return gemm_tiled_ok(kquant_gemm_type(type), repacked, x, n_rows, k, n_tokens);
 }
 
 size_t gemm_kquant_workspace_bytes(int type, size_t n_rows, size_t n_tokens, size_t k) {
   return al256(kquant_repacked_bytes(type, n_rows, k)) +
-         gemm_tiled_workspace_bytes(kquant_gemm_type(type), n_rows, n_tokens, kquant_gemm_k(type, k));
+         gemm_tiled_workspace_bytes(kquant_gemm_type(type), n_rows, n_tokens, k);
 }
 
+// xb: the activations are bfloat16 (at x).
 int launch_gemm_kquant(int type, const void* w, size_t n_rows, size_t k, const float* x, size_t n_tokens,
-                       float* y, void* workspace, hipStream_t s) {
+                       float* y, void* workspace, hipStream_t s, bool xb) {
   const int it = kquant_gemm_type(type);
-  const size_t kk = kquant_gemm_k(type, k);
   char* rp = static_cast<char*>(workspace);
-  const TiledWs t = tiled_ws(it, n_rows, kk, n_tokens, rp + al256(kquant_repacked_bytes(type, n_rows, k)));
+  const TiledWs t = tiled_ws(it, n_rows, k, n_tokens, rp + al256(kquant_repacked_bytes(type, n_rows, k)));
   // a handle's copy prepared once (wh_weight_prepare_prefill), else a conversion per call
   const char* src = static_cast<const char*>(prepared_kquant(w, type, n_rows, k));
   int st = src ? WH_OK : launch_repack_kquant(type, w, n_rows, k, rp, s);
   if (!src) src = rp;
-  if (!st) st = tiled_pack<kPackPlain>(it, t, x, nullptr, nullptr, 0.f, n_tokens, kk, k, s);
+  if (!st) st = xb ? tiled_pack<kPackPlain, true>(it, t, x, nullptr, nullptr, 0.f, n_tokens, k, s)
+                   : tiled_pack<kPackPlain>(it, t, x, nullptr, nullptr, 0.f, n_tokens, k, s);
   if (st) return st;
-  return kquant_run(type, src, n_rows, k, n_tokens, t, y, s);
+  return tiled_run(it, src, n_rows, k, n_tokens, t, y, s, 0, /*lo=*/!xb);
 }
 
+// Whether gate and up run as one GEMM: its tiles fill the CUs without split-K.
+static bool ffn_one_pass(int it, size_t n_ff, size_t n_tokens, size_t hidden) {
+  return gemm_tiled_splits(it, 2 * n_ff, n_tokens, hidden) == 1;
+}
+
+// Gate and up in one pass need both matrices repacked at the same time.
 size_t ffn_kquant_workspace_bytes(int type, size_t hidden, size_t n_ff, size_t n_tokens) {
   const int it = kquant_gemm_type(type);
-  const size_t r1 = kquant_repacked_bytes(type, n_ff, hidden), r2 = kquant_repacked_bytes(type, hidden, n_ff);
-  const size_t t1 = gemm_tiled_workspace_bytes(it, n_ff, n_tokens, kquant_gemm_k(type, hidden));
-  const size_t t2 = gemm_tiled_workspace_bytes(it, hidden, n_tokens, kquant_gemm_k(type, n_ff));
-  return al256(r1 > r2 ? r1 : r2) + (t1 > t2 ? t1 : t2);
+  const size_t r1 = al256(kquant_repacked_bytes(type, n_ff, hidden)) * (ffn_one_pass(it, n_ff, n_tokens, hidden) ? 2 : 1);
+  const size_t r2 = al256(kquant_repacked_bytes(type, hidden, n_ff));
+  const size_t t1 = gemm_tiled_workspace_bytes(it, n_ff, n_tokens, hidden);
+  const size_t t2 = gemm_tiled_workspace_bytes(it, hidden, n_tokens, n_ff);
+  return (r1 > r2 ? r1 : r2) + (t1 > t2 ? t1 : t2);
 }
 
 // The FFN for n_tokens rows on the tiled kernel: the RMSNorm of x is packed
@@ -1399,36 +1260,44 @@ int launch_ffn_tiled(int type, const void* gate, const void* up, const void* dow
                      const float* x, const float* gamma, float eps, size_t n_tokens, float* g, float* u, float* out,
                      void* workspace, size_t workspace_bytes, hipStream_t s) {
   if (is_kquant(type)) {
-    // one repacked matrix at a time in the front of the workspace (stream order
-    // keeps a GEMM's reads ahead of the next repack)
+    // the repacked matrices in the front of the workspace: gate and up side by
+    // side for one pass, else one at a time (stream order keeps a GEMM's reads
+    // ahead of the next repack)
     const int it = kquant_gemm_type(type);
-    const size_t H2 = kquant_gemm_k(type, hidden), F2 = kquant_gemm_k(type, n_ff);
-    const size_t r1 = kquant_repacked_bytes(type, n_ff, hidden), r2 = kquant_repacked_bytes(type, hidden, n_ff);
+    const bool one = ffn_one_pass(it, n_ff, n_tokens, hidden);
+    const size_t r1 = al256(kquant_repacked_bytes(type, n_ff, hidden)), r2 = al256(kquant_repacked_bytes(type, hidden, n_ff));
     char* rp = static_cast<char*>(workspace);
-    char* ws = rp + al256(r1 > r2 ? r1 : r2);
+    char* ws = rp + (r1 * (one ? 2 : 1) > r2 ? r1 * (one ? 2 : 1) : r2);
     if (!gemm_kquant_ok(type, gate, x, n_ff, hidden, n_tokens) || !aligned(up, 16) || !aligned(down, 16) ||
         !gemm_kquant_ok(type, down, g, hidden, n_ff, n_tokens) || !aligned(gamma, 16) || !aligned(u, 16) ||
         !aligned(workspace, 256) || workspace_bytes < ffn_kquant_workspace_bytes(type, hidden, n_ff, n_tokens))
       return WH_ERR_INVALID_SHAPE;
-    // each matrix: its handle's prepared copy, or converted into rp for this call
-    auto repacked = [&](const void* w, size_t rows, size_t k, const char** out_rp) -> int {
+    // each matrix: its handle's prepared copy, or converted into `at` for this call
+    auto repacked = [&](const void* w, size_t rows, size_t k, char* at, const char** out_rp) -> int {
       const char* pre = static_cast<const char*>(prepared_kquant(w, type, rows, k));
-      *out_rp = pre ? pre : rp;
-      return pre ? WH_OK : launch_repack_kquant(type, w, rows, k, rp, s);
+      *out_rp = pre ? pre : at;
+      return pre ? WH_OK : launch_repack_kquant(type, w, rows, k, at, s);
     };
-    const char* src = nullptr;
-    const TiledWs t1 = tiled_ws(it, n_ff, H2, n_tokens, ws);
-    int st = tiled_pack<kPackNorm>(it, t1, x, nullptr, gamma, eps, n_tokens, H2, hidden, s);
-    if (!st) st = repacked(gate, n_ff, hidden, &src);
-    if (!st) st = kquant_run(type, src, n_ff, hidden, n_tokens, t1, g, s, 0);
-    if (!st) st = repacked(up, n_ff, hidden, &src);
-    if (!st) st = kquant_run(type, src, n_ff, hidden, n_tokens, t1, u, s, 1);
+    const char *src = nullptr, *src2 = nullptr;
+    const TiledWs t1 = tiled_ws(it, n_ff, hidden, n_tokens, ws);
+    const TiledWs t2 = tiled_ws(it, hidden, n_ff, n_tokens, ws);
+    int st = tiled_pack<kPackNorm>(it, t1, x, nullptr, gamma, eps, n_tokens, hidden, s);
+    if (!st) st = repacked(gate, n_ff, hidden, rp, &src);
+    if (one) {
+      // h = silu(g) * u written by the epilogue (g holds h)
+      if (!st) st = repacked(up, n_ff, hidden, rp + r1, &src2);
+      if (!st) st = sb_run(it, reinterpret_cast<const uint8_t*>(src), reinterpret_cast<const uint8_t*>(src2), n_ff, hidden,
+                           n_tokens, t1, g, 1, 0, true, s);
+      if (!st) st = tiled_pack<kPackPlain>(it, t2, g, nullptr, nullptr, 0.f, n_tokens, n_ff, s);
+    } else {
+      if (!st) st = tiled_run(it, src, n_ff, hidden, n_tokens, t1, g, s, 0);
+      if (!st) st = repacked(up, n_ff, hidden, rp, &src);
+      if (!st) st = tiled_run(it, src, n_ff, hidden, n_tokens, t1, u, s, 1);
+      if (!st) st = tiled_pack<kPackSwiglu>(it, t2, g, u, nullptr, 0.f, n_tokens, n_ff, s);
+    }
+    if (!st) st = repacked(down, hidden, n_ff, rp, &src);
     if (st) return st;
-    const TiledWs t2 = tiled_ws(it, hidden, F2, n_tokens, ws);
-    st = tiled_pack<kPackSwiglu>(it, t2, g, u, nullptr, 0.f, n_tokens, F2, n_ff, s);
-    if (!st) st = repacked(down, hidden, n_ff, &src);
-    if (st) return st;
-    return kquant_run(type, src, hidden, n_ff, n_tokens, t2, out, s);
+    return tiled_run(it, src, hidden, n_ff, n_tokens, t2, out, s);
   }
   if (!gemm_tiled_ok(type, gate, x, n_ff, hidden, n_tokens) || !gemm_tiled_ok(type, up, x, n_ff, hidden, n_tokens) ||
       !gemm_tiled_ok(type, down, g, hidden, n_ff, n_tokens) || !aligned(gamma, 16) || !aligned(u, 16))
@@ -1437,10 +1306,10 @@ int launch_ffn_tiled(int type, const void* gate, const void* up, const void* dow
       workspace_bytes < gemm_tiled_workspace_bytes(type, hidden, n_tokens, n_ff))
     return WH_ERR_INVALID_SHAPE;
   const TiledWs t1 = tiled_ws(type, n_ff, hidden, n_tokens, workspace);
-  int st = tiled_pack<kPackNorm>(type, t1, x, nullptr, gamma, eps, n_tokens, hidden, hidden, s);
+  int st = tiled_pack<kPackNorm>(type, t1, x, nullptr, gamma, eps, n_tokens, hidden, s);
   if (st) return st;
   const TiledWs t2 = tiled_ws(type, hidden, n_ff, n_tokens, workspace);
-  if (gemm_tiled_splits(2 * n_ff, n_tokens, hidden) == 1) {
+  if (gemm_tiled_splits(type, 2 * n_ff, n_tokens, hidden) == 1) {
     // enough tiles without split-K: gate and up in one pass, h = silu(g) * u
     // written by its epilogue (g holds h), then packed for the down projection
     const uint8_t* gp = static_cast<const uint8_t*>(gate);
@@ -1451,11 +1320,11 @@ int launch_ffn_tiled(int type, const void* gate, const void* up, const void* dow
       case WH_TYPE_Q4_1: st = launch_ffn_typed<WH_TYPE_Q4_1>(gp, upp, n_ff, hidden, n_tokens, t1.frag, t1.rs, t1.bs, g, sk, s); break;
       default: st = launch_ffn_typed<WH_TYPE_Q8_0>(gp, upp, n_ff, hidden, n_tokens, t1.frag, t1.rs, t1.bs, g, sk, s); break;
     }
-    if (!st) st = tiled_pack<kPackPlain>(type, t2, g, nullptr, nullptr, 0.f, n_tokens, n_ff, n_ff, s);
+    if (!st) st = tiled_pack<kPackPlain>(type, t2, g, nullptr, nullptr, 0.f, n_tokens, n_ff, s);
   } else {
-    st = tiled_run(type, gate, n_ff, hidden, n_tokens, t1, g, s, nullptr, 0);
-    if (!st) st = tiled_run(type, up, n_ff, hidden, n_tokens, t1, u, s, nullptr, 1);
-    if (!st) st = tiled_pack<kPackSwiglu>(type, t2, g, u, nullptr, 0.f, n_tokens, n_ff, n_ff, s);
+    st = tiled_run(type, gate, n_ff, hidden, n_tokens, t1, g, s, 0);
+    if (!st) st = tiled_run(type, up, n_ff, hidden, n_tokens, t1, u, s, 1);
+    if (!st) st = tiled_pack<kPackSwiglu>(type, t2, g, u, nullptr, 0.f, n_tokens, n_ff, s);
   }
   if (st) return st;
   return tiled_run(type, down, hidden, n_ff, n_tokens, t2, out, s);

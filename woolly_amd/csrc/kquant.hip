@@ -143,95 +143,120 @@ __global__ __launch_bounds__(256) void kq_gemv_kernel(const uint8_t* __restrict_
 }
 
 // ------------------------------------------------------ prefill repacking
-// The tiled prefill GEMM takes 32-element blocks with one scale each, so a
-// K-quant matrix is rewritten once per call (same row order, same element
-// order within a row) into:
-//   Q4_K -> {f32 d * scale_j; u8 qs[16]} per 32 elements j (quants in Q4_0's
-//     nibble order: byte i holds element i low, element i + 16 high), and the
-//     super-block's dmin (its fp16 bits) in an [n_rows][q4f_dmin_stride(k)]
-//     table after the blocks, zero past the row's k / 256 super-blocks; the
-//     value (d * scale_j) * q + dmin is then the GEMM's d * q plus dmin times
-//     the super-block's activation sum;
-//   Q6_K -> {f32 (d * scale_j) / 64; i8 q[16] = q - 32} per 16 elements j
-//     (the GEMM pads each to a 32-element block, upper half zero).
-// The scale products are exact in f32 (11-bit times 6- or 8-bit integers).
-// Every thread writes one output block; 16-byte aligned input.
-__global__ __launch_bounds__(256) void kq_repack_q4k_kernel(const uint8_t* __restrict__ w, size_t n_groups,
-                                                            size_t groups_per_row, size_t n_rows,
-                                                            uint32_t* __restrict__ out, uint16_t* __restrict__ dmin_t,
-                                                            size_t dmin_stride) {
-  for (size_t gi = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; gi < n_groups;
-       gi += static_cast<size_t>(gridDim.x) * blockDim.x) {
-    const uint8_t* b = w + (gi >> 3) * 144;
-    const int j = static_cast<int>(gi & 7);
-    const float d = whd::f16_bits_to_f32(b16(b + 12));
-    const uint4 q = *reinterpret_cast<const uint4*>(b + 16 + 16 * j);  // elements 32j .. 32j + 31
-    const uint32_t qw[4] = {q.x, q.y, q.z, q.w};
-    uint32_t o[5];
-    o[0] = __float_as_uint(__fmul_rn(d, static_cast<float>(q4k_scale(b, j))));
-    // element e is nibble e & 1 of byte e >> 1; output byte 2m = lo(byte m) |
-    // lo(byte m + 8) << 4, byte 2m + 1 = hi(byte m) | hi(byte m + 8) << 4
-#pragma unroll
-    for (int c = 0; c < 4; c++) {
-      uint32_t v = 0;
-#pragma unroll
-      for (int t = 0; t < 2; t++) {
-        const int m = 2 * c + t;
-        const uint32_t lo = (qw[m >> 2] >> (8 * (m & 3))) & 0xFFu;
-        const uint32_t hi = (qw[(m + 8) >> 2] >> (8 * ((m + 8) & 3))) & 0xFFu;
-        const uint32_t b0 = (lo & 15u) | ((hi & 15u) << 4);
-        const uint32_t b1 = (lo >> 4) | (hi & 0xF0u);
-        v |= (b0 | (b1 << 8)) << (16 * t);
-      }
-      o[1 + c] = v;
-    }
-    uint32_t* dst = out + gi * 5;
-#pragma unroll
-    for (int c = 0; c < 5; c++) dst[c] = o[c];
-    if (j == 0) {
-      const size_t row = gi / groups_per_row, sb = (gi % groups_per_row) >> 3, nsb = groups_per_row >> 3;
-      uint16_t* tr = dmin_t + row * dmin_stride;
-      tr[sb] = b16(b + 14);
-      if (sb + 1 == nsb)  // the row's last super-block clears the padding
-        for (size_t z = nsb; z < dmin_stride; z++) tr[z] = 0;
-    }
-  }
+// A K-quant matrix is rewritten once per handle or call into the stage records
+// of the prefill GEMM (kGemmQ4S, kGemmQ6S in wh_common.hpp): the integer
+// quants and sub-block scales as they are, the scales and d as floats.  d is
+// exact (times a power of two); one that is inf or NaN becomes NaN, since the
+// reference's d * s * q is NaN for it wherever s or q is 0.
+__device__ __forceinline__ float record_d(uint32_t bits16, float p) {
+  const float d = whd::f16_bits_to_f32(bits16);
+  return __builtin_fmaf(d, 0.f, d) * p;
 }
 
-// Q6_K: a workgroup stages 32 consecutive blocks (6720 B, a 16-byte aligned
-// run) in LDS with coalesced 16-byte loads, then each thread rewrites halves.
-constexpr int kQ6Blocks = 32;
-__global__ __launch_bounds__(256) void kq_repack_q6k_kernel(const uint8_t* __restrict__ w, size_t n_blocks,
-                                                            uint32_t* __restrict__ out) {
-  __shared__ uint4 stage[kQ6Blocks * 210 / 16];
-  uint8_t* sb = reinterpret_cast<uint8_t*>(stage);
-  for (size_t b0 = static_cast<size_t>(blockIdx.x) * kQ6Blocks; b0 < n_blocks;
-       b0 += static_cast<size_t>(gridDim.x) * kQ6Blocks) {
-    const int nblk = static_cast<int>(n_blocks - b0 < kQ6Blocks ? n_blocks - b0 : kQ6Blocks);
-    const int bytes = nblk * 210;
-    const uint8_t* src = w + b0 * 210;
-    for (int i = threadIdx.x; i < bytes / 16; i += blockDim.x) stage[i] = reinterpret_cast<const uint4*>(src)[i];
-    for (int i = bytes / 16 * 16 + threadIdx.x; i < bytes; i += blockDim.x) sb[i] = src[i];
-    __syncthreads();
-    for (int h = threadIdx.x; h < nblk * 16; h += blockDim.x) {
-      const uint8_t* b = sb + (h >> 4) * 210;
-      const int j = h & 15;
-      const float d = whd::f16_bits_to_f32(b16(b + 208));
-      uint32_t o[5];
-      o[0] = __float_as_uint(__fmul_rn(__fmul_rn(d, static_cast<float>(b[192 + j])), 0.015625f));
-#pragma unroll
-      for (int c = 0; c < 4; c++) {
-        uint32_t v = 0;
-#pragma unroll
-        for (int t = 0; t < 4; t++) v |= ((q6k_quant(b, 16 * j + 4 * c + t) - 32u) & 0xFFu) << (8 * t);
-        o[1 + c] = v;
-      }
-      uint32_t* dst = out + (b0 * 16 + static_cast<size_t>(h)) * 5;
-#pragma unroll
-      for (int c = 0; c < 5; c++) dst[c] = o[c];
+// Q4_K: a workgroup stages one super-block of 64 rows in LDS (144-byte runs),
+// wave s forms their records of the super-block's stage s, and the records go
+// out through LDS as contiguous runs (read and written directly, 48 of 144 and
+// 8 of 40 bytes per lane and instruction, 14336 x 4096 took 17.1 us against
+// KQ4US).  16-byte aligned input.
+constexpr int kQ4Rows = 64;
+__global__ __launch_bounds__(256) void kq_repack_q4k_kernel(const uint8_t* __restrict__ w, int n_rows, int nsb,
+                                                            uint8_t* __restrict__ out, uint16_t* __restrict__ dmin_t,
+                                                            int dmin_stride) {
+  __shared__ uint4 stage[kQ4Rows * 9];
+  __shared__ uint2 rec2[4][kQ4Rows * 5];
+  const int sb = blockIdx.x, r0 = static_cast<int>(blockIdx.y) * kQ4Rows;
+  const int rows = min(kQ4Rows, n_rows - r0);
+  const int s = static_cast<int>(threadIdx.x) >> 6, row = static_cast<int>(threadIdx.x) & 63;
+  for (int i = threadIdx.x; i < 9 * rows; i += 256)
+    stage[i] = *reinterpret_cast<const uint4*>(w + (static_cast<size_t>(r0 + i / 9) * nsb + sb) * 144 + 16 * (i % 9));
+  __syncthreads();
+  // even quants of a dword into its low half, odd ones into the high half
+  auto split = [](uint32_t u) {
+    auto gather = [](uint32_t x) {
+      x = (x | (x >> 4)) & 0x00FF00FFu;
+      return (x | (x >> 8)) & 0xFFFFu;
+    };
+    return gather(u & 0x0F0F0F0Fu) | (gather((u >> 4) & 0x0F0F0F0Fu) << 16);
+  };
+  auto scale = [](uint32_t v) {
+    return static_cast<uint32_t>(__builtin_bit_cast(uint16_t, static_cast<_Float16>(static_cast<float>(v << 10))));
+  };
+  if (row < rows) {
+    const uint4 h = stage[9 * row], qa = stage[9 * row + 1 + 2 * s], qb = stage[9 * row + 2 + 2 * s];
+    // scales 2s, 2s + 1: bits 0..5 and 14..19 of the 24 bits at bit 24s
+    const uint32_t pr = s == 0 ? h.x : (s == 1 ? (h.x >> 24) | (h.y << 8) : (s == 2 ? (h.y >> 16) | (h.z << 16) : h.z >> 8));
+    uint2* rec = rec2[s] + 5 * row;
+    rec[0] = make_uint2(split(qa.x), split(qa.y));
+    rec[1] = make_uint2(split(qa.z), split(qa.w));
+    rec[2] = make_uint2(split(qb.x), split(qb.y));
+    rec[3] = make_uint2(split(qb.z), split(qb.w));
+    rec[4] = make_uint2(scale(pr & 63u) | (scale((pr >> 14) & 63u) << 16), __float_as_uint(record_d(h.w & 0xFFFFu, 16384.f)));
+    if (s == 0) {
+      uint16_t* tr = dmin_t + static_cast<size_t>(r0 + row) * dmin_stride;
+      tr[sb] = static_cast<uint16_t>(h.w >> 16);
+      if (sb + 1 == nsb)  // the row's last super-block clears the padding
+        for (int z = nsb; z < dmin_stride; z++) tr[z] = 0;
     }
-    __syncthreads();
   }
+  __syncthreads();
+  uint2* dst = reinterpret_cast<uint2*>(out + (static_cast<size_t>(4 * sb + s) * n_rows + r0) * 40);
+  for (int i = row; i < 5 * rows; i += 64) dst[i] = rec2[s][i];
+}
+
+// Q6_K: a workgroup stages one super-block of 32 rows in LDS (a wavefront per
+// row and load: the 210 bytes as dwords, which are only 2-byte aligned in
+// memory), each thread forms half a record: 32 elements share 16 bytes of ql
+// (element i and i + 16 the same byte) and 8 bytes of qh (9 for the upper half
+// of the block, whose bits start 2 higher and run into the next byte).  The
+// records go through LDS too, so that the stores are contiguous (80-byte
+// records stored as they are formed: 44 us for 14336 x 4096 against 35 us).
+constexpr int kQ6Rows = 32, kQ6Stride = 53;  // dwords per staged block
+__global__ __launch_bounds__(256) void kq_repack_q6k_kernel(const uint8_t* __restrict__ w, int n_rows, int nsb,
+                                                            uint8_t* __restrict__ out) {
+  __shared__ uint32_t stage[kQ6Rows * kQ6Stride];
+  __shared__ uint4 rec4[4][kQ6Rows * 5];
+  const int sb = blockIdx.x, r0 = static_cast<int>(blockIdx.y) * kQ6Rows;
+  const int rows = min(kQ6Rows, n_rows - r0);
+  const int wave = static_cast<int>(threadIdx.x) >> 6, lane = static_cast<int>(threadIdx.x) & 63;
+#pragma unroll
+  for (int i = 0; i < kQ6Rows / 4; i++) {
+    const int r = 4 * i + wave;
+    const uint8_t* b = w + (static_cast<size_t>(r0 + min(r, rows - 1)) * nsb + sb) * 210 + 4 * lane;
+    if (lane >= kQ6Stride) continue;
+    uint32_t v;
+    if (lane < kQ6Stride - 1) __builtin_memcpy(&v, b, 4);
+    else v = *reinterpret_cast<const uint16_t*>(b);  // the block's last two bytes: d
+    stage[r * kQ6Stride + lane] = v;
+  }
+  __syncthreads();
+  const int s = wave, r = lane >> 1, half = lane & 1;
+  {
+    const uint32_t* b = stage + r * kQ6Stride;
+    const bool upper = s >= 2;
+    const int grp = 2 * s + half;               // elements 32 grp ..
+    uint32_t h[3] = {b[32 + 2 * grp], b[33 + 2 * grp], grp == 7 ? 0u : b[34 + 2 * grp]};
+    uint32_t q[8];
+#pragma unroll
+    for (int c = 0; c < 8; c++) {
+      const uint32_t nib = (b[4 * grp + (c & 3)] >> (upper ? 4 : 0)) & 0x0F0F0F0Fu;
+      // byte c of h with the byte behind it, the pairs of bits from bit 0 (2)
+      const uint32_t two = __builtin_amdgcn_alignbit(h[c / 4 + 1], h[c / 4], 8 * (c & 3)) >> (upper ? 2 : 0);
+      q[c] = nib | (two & 3u) << 4 | (two & 0xCu) << 10 | (two & 0x30u) << 16 | (two & 0xC0u) << 22;
+    }
+    uint4* rec = rec4[s] + 5 * r;
+    rec[2 * half] = make_uint4(q[0], q[1], q[2], q[3]);
+    rec[2 * half + 1] = make_uint4(q[4], q[5], q[6], q[7]);
+    const uint32_t sc = b[48 + s] >> (16 * half);  // scales 4s + 2 half, + 1
+    auto scale = [](uint32_t v) {
+      return static_cast<uint32_t>(__builtin_bit_cast(uint16_t, static_cast<_Float16>(static_cast<float>(v & 0xFFu))));
+    };
+    uint32_t* meta = reinterpret_cast<uint32_t*>(rec + 4);
+    meta[half] = scale(sc) | (scale(sc >> 8) << 16);
+    meta[2 + half] = half ? 0u : __float_as_uint(record_d(b[52] & 0xFFFFu, 0.015625f));
+  }
+  __syncthreads();
+  uint4* dst = reinterpret_cast<uint4*>(out + (static_cast<size_t>(4 * sb + s) * n_rows + r0) * 80);
+  for (int i = lane; i < 5 * rows; i += 64) dst[i] = rec4[s][i];
 }
 
 unsigned kq_grid(size_t work, unsigned per_block) {
@@ -276,14 +301,13 @@ int launch_gemv_kquant(int type, const void* w, const float* x, float* y, size_t
 int launch_repack_kquant(int type, const void* w, size_t n_rows, size_t k, void* out, hipStream_t s) {
   if (n_rows == 0 || k == 0) return WH_OK;
   const uint8_t* p = static_cast<const uint8_t*>(w);
-  uint32_t* o = static_cast<uint32_t*>(out);
+  uint8_t* o = static_cast<uint8_t*>(out);
+  const int rows = static_cast<int>(n_rows), nsb = static_cast<int>(k / 256);
   if (type == WH_TYPE_Q4_K) {
-    const size_t n = n_rows * (k / 32);
-    uint16_t* dmin_t = reinterpret_cast<uint16_t*>(static_cast<char*>(out) + n * 20);
-    kq_repack_q4k_kernel<<<kq_grid(n, 256), 256, 0, s>>>(p, n, k / 32, n_rows, o, dmin_t, q4f_dmin_stride(k));
+    uint16_t* dmin_t = reinterpret_cast<uint16_t*>(o + n_rows * (k / 64) * 40);
+    kq_repack_q4k_kernel<<<dim3(nsb, (rows + kQ4Rows - 1) / kQ4Rows), 256, 0, s>>>(p, rows, nsb, o, dmin_t, static_cast<int>(q4s_dmin_stride(k)));
   } else {
-    const size_t n = n_rows * (k / 256);
-    kq_repack_q6k_kernel<<<kq_grid(n, kQ6Blocks), 256, 0, s>>>(p, n, o);
+    kq_repack_q6k_kernel<<<dim3(nsb, (rows + kQ6Rows - 1) / kQ6Rows), 256, 0, s>>>(p, rows, nsb, o);
   }
   WH_LAUNCH_CHECK("k-quant repack kernel launch");
   return WH_OK;

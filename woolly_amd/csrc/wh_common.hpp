@@ -68,23 +68,22 @@ inline bool is_block_type(int type) {
 // The 256-element K-quant formats.
 inline bool is_kquant(int type) { return type == WH_TYPE_Q4_K || type == WH_TYPE_Q6_K; }
 
-// Block formats of the tiled prefill GEMM that K-quant matrices are repacked
-// into (internal ids, never seen at the C ABI):
-//   kGemmQ4F {f32 d; u8 qs[16]}: 32 elements d * q, Q4_0 nibble order, followed
-//            by the super-blocks' dmin as fp16 [n_rows][q4f_dmin_stride(k)]
-//            (zeros past k / 256; the GEMM's epilogue adds dmin * sum(x) per
-//            super-block, as matrix-core products over 32 super-blocks)
-//   kGemmQ8H {f32 d; i8 q[16]}: 16 elements d * q, which the GEMM reads as a
-//            32-element block whose upper half is zero (activations packed to match)
-constexpr int kGemmQ4F = 256, kGemmQ8H = 257;
-inline int kquant_gemm_type(int type) { return type == WH_TYPE_Q4_K ? kGemmQ4F : kGemmQ8H; }
-// The GEMM's reduction length for a K-quant row of k elements.
-inline size_t kquant_gemm_k(int type, size_t k) { return type == WH_TYPE_Q4_K ? k : 2 * k; }
-// Super-blocks per row of kGemmQ4F's dmin table: k / 256 rounded up to 8
+// Formats of the prefill GEMM that K-quant matrices are repacked into
+// (internal ids, never seen at the C ABI): stage records, [k / 64][n_rows] of
+//   kGemmQ4S 40 B: 32 quant bytes (64 elements; dword i holds elements 8i ..
+//            8i + 7, the even ones in its low half), f16 s 2^10 of the two
+//            32-element groups, f32 d 2^14; behind the records the
+//            super-blocks' dmin as fp16 [n_rows][q4s_dmin_stride(k)] (zeros
+//            past k / 256)
+//   kGemmQ6S 80 B: 64 quant bytes (0..63), f16 s of the four 16-element
+//            groups, f32 d / 64, 4 unused bytes
+constexpr int kGemmQ4S = 256, kGemmQ6S = 257;
+inline int kquant_gemm_type(int type) { return type == WH_TYPE_Q4_K ? kGemmQ4S : kGemmQ6S; }
+// Super-blocks per row of kGemmQ4S's dmin table: k / 256 rounded up to 8
 // (16-byte rows).
-inline size_t q4f_dmin_stride(size_t k) { return (k / 256 + 7) / 8 * 8; }
+inline size_t q4s_dmin_stride(size_t k) { return (k / 256 + 7) / 8 * 8; }
 inline size_t kquant_repacked_bytes(int type, size_t n_rows, size_t k) {
-  return n_rows * (type == WH_TYPE_Q4_K ? k / 32 * 20 + q4f_dmin_stride(k) * 2 : k / 16 * 20);
+  return n_rows * (type == WH_TYPE_Q4_K ? k / 64 * 40 + q4s_dmin_stride(k) * 2 : k / 64 * 80);
 }
 // Rewrites a Q4_K / Q6_K matrix (n_rows x k, 16-byte aligned) into the format above (kquant.hip).
 int launch_repack_kquant(int type, const void* w, size_t n_rows, size_t k, void* out, hipStream_t stream);
@@ -190,12 +189,12 @@ int launch_gemm_tiled_bf16(int type, const void* w, size_t n_rows, size_t k, con
                            float* y, void* workspace, hipStream_t s);
 // bfloat16 -> f32 (exact), n elements.
 int launch_bf16_to_f32(const uint16_t* x, size_t n, float* out, hipStream_t s);
-// Q4_K / Q6_K on the tiled kernel: the matrix repacked into the front of the
-// workspace, then the GEMM.
+// Q4_K / Q6_K (gemm_sb.hpp): the matrix repacked into the front of the
+// workspace, then the GEMM; xb: x holds bfloat16 values.
 bool gemm_kquant_ok(int type, const void* w, const float* x, size_t n_rows, size_t k, size_t n_tokens);
 size_t gemm_kquant_workspace_bytes(int type, size_t n_rows, size_t n_tokens, size_t k);
 int launch_gemm_kquant(int type, const void* w, size_t n_rows, size_t k, const float* x, size_t n_tokens,
-                       float* y, void* workspace, hipStream_t stream);
+                       float* y, void* workspace, hipStream_t stream, bool xb = false);
 // Workspace of launch_ffn_tiled beyond its g / u scratch, for a K-quant FFN.
 size_t ffn_kquant_workspace_bytes(int type, size_t hidden, size_t n_ff, size_t n_tokens);
 // FFN for more than kGemvTokenLimit tokens on the tiled kernel, with the
