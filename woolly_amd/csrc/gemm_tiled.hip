@@ -103,15 +103,17 @@ template <int TYPE, int BM>
 constexpr int per_stage() {
   return (SB * TCfg<BM>::FPB + TWAVES - 1) / TWAVES + b_dma_per_wave<TYPE>();
 }
-// Ring depth: as many stages as 160 KiB of LDS holds, 3 to 8 (a deeper ring
-// keeps more weight bytes in flight where a stage is small), with the copies
-// of the stages in flight behind the one awaited countable by vmcnt (< 64).
+// Ring depth: 3 or 4 stages in the 160 KiB of LDS, with the copies of the
+// stages in flight behind the one awaited countable by vmcnt (< 64).  A deeper
+// ring (the small token tiles would fit 8) only lengthens the fill before the
+// first product: Q4_0 14336 x 4096 at 32 / 64 tokens takes 27.5 / 38.3 us with
+// up to 8, 26.7 / 36.1 with 5, 25.5 / 35.1 with 4, 25.8 / 34.8 with 3.
 template <int TYPE, int BM>
 constexpr int nstage() {
   constexpr int n = 160 * 1024 / stage_bytes<TYPE, BM>();
   constexpr int v = 2 + 63 / per_stage<TYPE, BM>();
   constexpr int m = n < v ? n : v;
-  return m < 3 ? 3 : (m > 8 ? 8 : m);
+  return m < 3 ? 3 : (m > 4 ? 4 : m);
 }
 template <int TYPE, int BM>
 constexpr size_t tiled_lds_bytes() { return static_cast<size_t>(nstage<TYPE, BM>()) * stage_bytes<TYPE, BM>(); }
