@@ -485,7 +485,8 @@ KERNEL_SOURCE_GROUPS = {
     "gemv_mt": (_C + "gemv_mt.hpp", _C + "gemv_mfma_dev.hpp", _C + "gemv_mt_q4_0.hip", _C + "gemv_mt_q4_1.hip",
                 _C + "gemv_mt_q8_0.hip", _C + "gemv_mt_q4_k.hip", _C + "gemv_mt_q6_k.hip") + _COMMON,
     # tiled prefill GEMM, its packing, the K-quant conversion, the fallbacks
-    "gemm": (_C + "gemm_tiled.hip", _C + "gemm.hip", _C + "kquant.hip", _C + "elementwise.hip") + _COMMON,
+    "gemm": (_C + "gemm_tiled.hip", _C + "gemm_sb.hpp", _C + "gemm_sb_q4.hip", _C + "gemm_sb_q6.hip", _C + "gemm_sb_api.hpp",
+             _C + "gemm_dev.hpp", _C + "gemm.hip", _C + "kquant.hip", _C + "elementwise.hip") + _COMMON,
     "attention": (_C + "attention.hip",) + _COMMON,
 }
 # the decode step launches kernels of every group above and of decode.hip / embed.hip

@@ -183,9 +183,8 @@ def test_kquant_mfma_nonfinite_and_zero_chunks(gpu, orc, t):
 
 
 # ---------------------------------------------------------------- prefill
-# More than two tokens: the matrix is repacked into 32-element blocks with f32
-# scales (Q4_K: (d * scale) q + dmin; Q6_K: 16-element halves, (d * scale / 64)
-# (q - 32), padded to 32 with zeros) and multiplied on the tiled MFMA kernel.
+# More than 16 tokens: the matrix is repacked into stage records of 64 elements
+# (quants, sub-block scales in fp16, d in f32) and multiplied on the matrix cores.
 # (m, n, k): one to 56 super-blocks per row, ragged token and row counts,
 # token tiles of 16 .. 128, split-K
 KQ_MATMUL = [(3, 300, 4096), (8, 1024, 2048), (17, 768, 256), (64, 129, 4096), (130, 200, 512),
@@ -196,7 +195,9 @@ KQ_MATMUL = [(3, 300, 4096), (8, 1024, 2048), (17, 768, 256), (64, 129, 4096), (
 # that start 8 bytes off a 16-byte boundary), one super-block per row, and
 # tiles shared by two workgroups of the stream-K grid (14337 and 5000 rows)
 KQ_EDGES = [(17, 1, 256), (32, 255, 256), (33, 257, 768), (64, 301, 512), (65, 513, 2304), (128, 1001, 1024),
-            (129, 14337, 256), (257, 5000, 1280)]
+            (129, 14337, 256), (257, 5000, 1280),
+            # 7 and 8 super-blocks per workgroup and tile: products accumulated over 64 and over 128 elements
+            (300, 2560, 14336), (300, 2561, 14336)]
 
 
 @pytest.mark.parametrize("t", [Q4_K, Q6_K])

@@ -6,10 +6,10 @@
 //   Q6_K  w = (d / 64) (s_j (q - 32)) s_j 8 bits, q 6 bits: |..| <= 8160
 // so the sub-block scale s_j goes into the fp16 weight operand (Q4_K: the
 // product is an fp16 exactly; Q6_K: hi = fp16(s_j (q - 32)) and the exact rest
-// lo) and the matrix cores accumulate a whole super-block, 8 steps of 32
-// elements, before one f32 FMA per output applies d.  With 32-element blocks
-// and a scale per block that FMA comes once per step, which made the vector
-// ALU the bound (3.4 VALU operations per MFMA; here 1.9 for Q4_K), and Q6_K's
+// lo) and the matrix cores accumulate 64 or 128 elements (sb_chain) before one
+// f32 FMA per output applies d.  With 32-element blocks and a scale per block
+// that FMA comes once per step and the scale's product with it, which made the
+// vector ALU the bound (3.4 VALU operations per MFMA), and Q6_K's
 // 16-element groups had to be padded with zeros to 32 (four products per
 // 32 elements; here three: x_lo w_hi, x_hi w_hi, x_hi w_lo; the x_lo w_lo
 // left out is below 2^-23 of x w, and x itself carries 22 bits).
@@ -39,6 +39,8 @@
 #include "gemm_dev.hpp"
 #include "gemm_sb_api.hpp"
 
+#include <algorithm>
+
 namespace {
 
 template <int BM>
@@ -50,6 +52,19 @@ struct SbCfg {
 
 template <int TYPE>
 constexpr int sb_rec() { return TYPE == wh::kGemmQ4S ? 40 : 80; }  // bytes per row and stage
+
+// Stages after the first that the matrix cores accumulate before d is applied
+// (0: 64 elements, 1: 128), for the sb super-blocks that a workgroup
+// sums per tile.  An MFMA rounds its
+// products at the size of its C operand, so a long chain loses more than the f32
+// FMAs of a short one; in a long sum the FMAs do, since the sum outgrows the
+// chain.  A step's products with an x_lo or w_lo come first, while C is small.
+// Error against 64 bits, Q4_K 14336 x 4096: chains of 256, x_hi first, 2.8e-7
+// at M=32, 2.9e-7 at M=128, 3.0e-7 at M=512; of 64, x_lo first, 2.0e-7, 2.3e-7,
+// 2.7e-7; of 128 2.4e-7 at M=128, 2.6e-7 at M=512 (a workgroup
+// sums 4 super-blocks at M=128, 14 at M=512).  Of 32 worse again: 2.2e-7 at M=32.  Time at M=512: 127
+// us with 64, 120.6 with 128; at M=128 55.1 and 53.5.
+inline int sb_chain(int bm, int sb) { return bm == 128 && sb >= 8 ? 1 : 0; }
 
 template <int TYPE, int BM, bool LO>
 struct SbStage {
@@ -82,7 +97,8 @@ __global__ __launch_bounds__(TWAVES * 64, 1) void gemm_sb_kernel(
     const uint8_t* __restrict__ W, const uint8_t* __restrict__ W2, const _Float16* __restrict__ frag,
     const float* __restrict__ rscale, const float* __restrict__ bsum, float* __restrict__ y, int n_tokens, int n_rows,
     int nsb, int sb_per_split, int tiles_n, int n_tiles, uint32_t* __restrict__ sk_flags, float* __restrict__ sk_part,
-    int sk_upw, int sk_sub, uint32_t sk_wait) {
+    int sk_upw, int sk_sub, uint32_t sk_wait,
+    int chain) {
   using C = SbCfg<BM>;
   using S = SbStage<TYPE, BM, LO>;
   constexpr int IT = C::IT, NT = C::NT, REC = sb_rec<TYPE>(), N = S::N;
@@ -186,7 +202,7 @@ __global__ __launch_bounds__(TWAVES * 64, 1) void gemm_sb_kernel(
   half8 ah[IT], al[IT], bw[NT], bl[NT];
   uint2 rq[NT];          // quants: Q4_K both steps of the stage, Q6_K one step
   half2v sc[NT];         // the lane's scale of the stage in both halves
-  float dn[NT];          // d of the super-block whose products are pending
+  float dn[NT];          // d of the chain whose products are pending
   auto read_a = [&](const uint8_t* slot, int t, int limb, half8 (&dst)[IT]) {
 #pragma unroll
     for (int i = 0; i < IT; i++)
@@ -246,7 +262,7 @@ __global__ __launch_bounds__(TWAVES * 64, 1) void gemm_sb_kernel(
       bl[n][2 * c + 1] = r[1];
     }
   };
-  // acc += d cc of row group n, whose next super-block starts from zero
+  // acc += d cc of row group n, whose next chain starts from zero
   auto apply = [&](int n, float d) {
 #pragma unroll
     for (int i = 0; i < IT; i++)
@@ -290,7 +306,7 @@ __global__ __launch_bounds__(TWAVES * 64, 1) void gemm_sb_kernel(
   read_q(smem, 0);
   read_s(smem);
   if constexpr (Q4) {
-    read_a(smem, 0, 0, ah);
+    read_a(smem, 0, 1, al);
     form(0, 0);
     if constexpr (NT > 2) form(1, 0);
   } else {
@@ -306,7 +322,9 @@ __global__ __launch_bounds__(TWAVES * 64, 1) void gemm_sb_kernel(
       const uint8_t* slot = smem + cur * S::BYTES;
       const int nxt = cur + 1 == N ? 0 : cur + 1;
       const uint8_t* nslot = smem + nxt * S::BYTES;
-      const bool head = (st & 3) == 0, tail = (st & 3) == 3;  // first / last stage of a super-block
+      // first / last stage of a chain; the branch stays: straight through, the
+      // 128-token body spills
+      const bool head = (st & chain) == 0, tail = (st & chain) == chain;
       // behind the last read of the stage's slot: the next stage landed
       // (every wave's copies), then the slot is refilled
       auto turn = [&]() {
@@ -320,13 +338,13 @@ __global__ __launch_bounds__(TWAVES * 64, 1) void gemm_sb_kernel(
       for (int t = 0; t < 2; t++) {
         const bool zero = head && t == 0, last = tail && t == 1;
         if constexpr (Q4) {
-          // phase hi: x_lo read; the weights of the step's later row groups
-          if constexpr (LO) read_a(slot, t, 1, al);
+          // phase x_lo (x_hi without LO): x_hi read; the weights of the step's later row groups
+          if constexpr (LO) read_a(slot, t, 0, ah);
           if (last) read_d(slot);
 #pragma unroll
           for (int n = 0; n < NT; n++) {
 #pragma unroll
-            for (int i = 0; i < IT; i++) mma(i, n, ah[i], bw[n]);
+            for (int i = 0; i < IT; i++) mma(i, n, al[i], bw[n]);
             if (zero && n == 0) apply(NT - 1, dn[NT - 1]);
             if (NT > 2 && n < 2) form(n + 2, t);
             if (NT == 2 && n == 0) form(1, t);
@@ -342,8 +360,8 @@ __global__ __launch_bounds__(TWAVES * 64, 1) void gemm_sb_kernel(
           for (int n = 0; n < NT; n++) {
 #pragma unroll
             for (int i = 0; i < IT; i++)
-              if constexpr (LO) mma(i, n, al[i], bw[n]);
-            if (n == 0) read_a(t ? nslot : slot, t ^ 1, 0, ah);
+              if constexpr (LO) mma(i, n, ah[i], bw[n]);
+            if (n == 0) read_a(t ? nslot : slot, t ^ 1, 1, al);
             if (last && n > 0) apply(n - 1, dn[n - 1]);
             if (NT > 2 && n >= 2) form(n - 2, t ^ 1);
             if (NT == 2 && n == 1) form(0, t ^ 1);
@@ -364,11 +382,11 @@ __global__ __launch_bounds__(TWAVES * 64, 1) void gemm_sb_kernel(
             __builtin_amdgcn_sched_barrier(0);
           }
           if (t == 1) turn();
-          // phase x_hi w_hi: the later w_lo formed, the next quants read
+          // phase x_hi w_lo: the later w_lo formed, the next quants read
 #pragma unroll
           for (int n = 0; n < NT; n++) {
 #pragma unroll
-            for (int i = 0; i < IT; i++) mma(i, n, ah[i], bw[n]);
+            for (int i = 0; i < IT; i++) mma(i, n, ah[i], bl[n]);
             if (n < NT / 2) form_lo(n + NT / 2);
             if (n == NT / 2) {
               read_q(t ? nslot : slot, t ^ 1);
@@ -376,11 +394,11 @@ __global__ __launch_bounds__(TWAVES * 64, 1) void gemm_sb_kernel(
             }
             __builtin_amdgcn_sched_barrier(0);
           }
-          // phase x_hi w_lo: the next x_lo read, the first w_hi formed
+          // phase x_hi w_hi: the next x_lo read, the next step's first w_hi formed
 #pragma unroll
           for (int n = 0; n < NT; n++) {
 #pragma unroll
-            for (int i = 0; i < IT; i++) mma(i, n, ah[i], bl[n]);
+            for (int i = 0; i < IT; i++) mma(i, n, ah[i], bw[n]);
             if (LO && n == 0) read_a(t ? nslot : slot, t ^ 1, 1, al);
             if (last && n > 0) apply(n - 1, dn[n - 1]);
             if (n >= NT / 2) form(n - NT / 2, t ^ 1);
@@ -554,9 +572,10 @@ int sb_launch(const wh::SbGemm& a, hipStream_t s) {
   WH_ENSURE_LDS(lds, &gemm_sb_kernel<TYPE, BM, FFNP, SK, LO>);
   const dim3 grid(static_cast<unsigned>(SK ? a.sk_g : n_tiles), static_cast<unsigned>(SK ? 1 : a.splits));
   const int upw = SK ? (n_tiles * nsb + a.sk_g - 1) / a.sk_g : 0;
+  const int sbps = (nsb + a.splits - 1) / a.splits;
   gemm_sb_kernel<TYPE, BM, FFNP, SK, LO><<<grid, TWAVES * 64, lds, s>>>(
-      a.w, a.w2, a.frag, a.rs, a.bs, a.y, a.n_tokens, a.n_rows, nsb, (nsb + a.splits - 1) / a.splits, tiles_n, n_tiles,
-      a.sk_flags, a.sk_part, upw, a.sk_sub, a.sk_wait);
+      a.w, a.w2, a.frag, a.rs, a.bs, a.y, a.n_tokens, a.n_rows, nsb, sbps, tiles_n, n_tiles,
+      a.sk_flags, a.sk_part, upw, a.sk_sub, a.sk_wait, sb_chain(BM, SK ? std::min(nsb, upw) : sbps));
   WH_LAUNCH_CHECK("k-quant gemm kernel launch");
   return WH_OK;
 }
