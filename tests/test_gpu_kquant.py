@@ -262,6 +262,22 @@ def test_kquant_matmul_parity(gpu, orc, t, m, n, k):
     assert r <= 1e-4 and a <= 1e-3
 
 
+@pytest.mark.parametrize("t,rows_per_group", [(Q4_K, 64), (Q6_K, 32)])
+def test_kquant_repack_many_row_groups(gpu, t, rows_per_group):
+    """A matrix with more row groups than a grid has in y (65535), one
+    super-block per row: its last rows give the bits of the same rows alone."""
+    m, k, base = 17, 256, 1024
+    n = rows_per_group * 65536 + 37
+    print(f"[case] kquant repack type={t} n={n}", flush=True)
+    part = synth.quantized_weight(t, base, k, seed=600 + t).reshape(base, TS[t])
+    w = part[np.arange(n) % base]
+    x = synth.activations(m * k, seed=601).reshape(m, k)
+    last = np.arange(n - base, n)
+    got = kq_matmul(t, w.reshape(-1), x, m, n, k)
+    assert same(np.ascontiguousarray(got[:, last]), kq_matmul(t, w[last].reshape(-1), x, m, base, k))
+    assert same(np.ascontiguousarray(got[:, :base]), kq_matmul(t, part.reshape(-1), x, m, base, k))
+
+
 @pytest.mark.parametrize("t", [Q4_K, Q6_K])
 def test_kquant_matmul_matches_gemv(gpu, t):
     """The tiled path (5 tokens) and the per-token GEMV agree on every token."""

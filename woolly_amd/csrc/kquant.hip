@@ -159,12 +159,12 @@ __device__ __forceinline__ float record_d(uint32_t bits16, float p) {
 // 8 of 40 bytes per lane and instruction, 14336 x 4096 took 17.1 us against
 // KQ4US).  16-byte aligned input.
 constexpr int kQ4Rows = 64;
-__global__ __launch_bounds__(256) void kq_repack_q4k_kernel(const uint8_t* __restrict__ w, int n_rows, int nsb,
+__global__ __launch_bounds__(256) void kq_repack_q4k_kernel(const uint8_t* __restrict__ w, int n_rows, unsigned nsb,
                                                             uint8_t* __restrict__ out, uint16_t* __restrict__ dmin_t,
                                                             int dmin_stride) {
   __shared__ uint4 stage[kQ4Rows * 9];
   __shared__ uint2 rec2[4][kQ4Rows * 5];
-  const int sb = blockIdx.x, r0 = static_cast<int>(blockIdx.y) * kQ4Rows;
+  const int sb = static_cast<int>(blockIdx.x % nsb), r0 = static_cast<int>(blockIdx.x / nsb) * kQ4Rows;
   const int rows = min(kQ4Rows, n_rows - r0);
   const int s = static_cast<int>(threadIdx.x) >> 6, row = static_cast<int>(threadIdx.x) & 63;
   for (int i = threadIdx.x; i < 9 * rows; i += 256)
@@ -194,8 +194,8 @@ __global__ __launch_bounds__(256) void kq_repack_q4k_kernel(const uint8_t* __res
     if (s == 0) {
       uint16_t* tr = dmin_t + static_cast<size_t>(r0 + row) * dmin_stride;
       tr[sb] = static_cast<uint16_t>(h.w >> 16);
-      if (sb + 1 == nsb)  // the row's last super-block clears the padding
-        for (int z = nsb; z < dmin_stride; z++) tr[z] = 0;
+      if (sb + 1 == static_cast<int>(nsb))  // the row's last super-block clears the padding
+        for (int z = static_cast<int>(nsb); z < dmin_stride; z++) tr[z] = 0;
     }
   }
   __syncthreads();
@@ -211,11 +211,11 @@ __global__ __launch_bounds__(256) void kq_repack_q4k_kernel(const uint8_t* __res
 // records go through LDS too, so that the stores are contiguous (80-byte
 // records stored as they are formed: 44 us for 14336 x 4096 against 35 us).
 constexpr int kQ6Rows = 32, kQ6Stride = 53;  // dwords per staged block
-__global__ __launch_bounds__(256) void kq_repack_q6k_kernel(const uint8_t* __restrict__ w, int n_rows, int nsb,
+__global__ __launch_bounds__(256) void kq_repack_q6k_kernel(const uint8_t* __restrict__ w, int n_rows, unsigned nsb,
                                                             uint8_t* __restrict__ out) {
   __shared__ uint32_t stage[kQ6Rows * kQ6Stride];
   __shared__ uint4 rec4[4][kQ6Rows * 5];
-  const int sb = blockIdx.x, r0 = static_cast<int>(blockIdx.y) * kQ6Rows;
+  const int sb = static_cast<int>(blockIdx.x % nsb), r0 = static_cast<int>(blockIdx.x / nsb) * kQ6Rows;
   const int rows = min(kQ6Rows, n_rows - r0);
   const int wave = static_cast<int>(threadIdx.x) >> 6, lane = static_cast<int>(threadIdx.x) & 63;
 #pragma unroll
@@ -302,12 +302,15 @@ int launch_repack_kquant(int type, const void* w, size_t n_rows, size_t k, void*
   if (n_rows == 0 || k == 0) return WH_OK;
   const uint8_t* p = static_cast<const uint8_t*>(w);
   uint8_t* o = static_cast<uint8_t*>(out);
-  const int rows = static_cast<int>(n_rows), nsb = static_cast<int>(k / 256);
+  const int rows = static_cast<int>(n_rows);
+  // super-blocks and row groups in x, the one grid dimension beyond 65535
+  const unsigned nsb = static_cast<unsigned>(k / 256);
+  auto grid = [&](int group) { return static_cast<unsigned>(nsb * ((n_rows + group - 1) / group)); };
   if (type == WH_TYPE_Q4_K) {
     uint16_t* dmin_t = reinterpret_cast<uint16_t*>(o + n_rows * (k / 64) * 40);
-    kq_repack_q4k_kernel<<<dim3(nsb, (rows + kQ4Rows - 1) / kQ4Rows), 256, 0, s>>>(p, rows, nsb, o, dmin_t, static_cast<int>(q4s_dmin_stride(k)));
+    kq_repack_q4k_kernel<<<grid(kQ4Rows), 256, 0, s>>>(p, rows, nsb, o, dmin_t, static_cast<int>(q4s_dmin_stride(k)));
   } else {
-    kq_repack_q6k_kernel<<<dim3(nsb, (rows + kQ6Rows - 1) / kQ6Rows), 256, 0, s>>>(p, rows, nsb, o);
+    kq_repack_q6k_kernel<<<grid(kQ6Rows), 256, 0, s>>>(p, rows, nsb, o);
   }
   WH_LAUNCH_CHECK("k-quant repack kernel launch");
   return WH_OK;
