@@ -45,15 +45,16 @@ def test_kquant_dequant_bit_exact(gpu, orc, t, n):
 
 
 @pytest.mark.parametrize("t", [Q4_K, Q6_K])
-@pytest.mark.parametrize("off", [0, 4])
+@pytest.mark.parametrize("doff,off", [(0, 0), (4, 4), (0, 4), (4, 0), (2, 0), (1, 0)])
 @pytest.mark.parametrize("blocks,tail", [(8192, 0), (8193, 0), (16384, 0), (16385, -3), (24577, -1)])
-def test_kquant_dequant_passes(gpu, orc, t, off, blocks, tail):
+def test_kquant_dequant_passes(gpu, orc, t, doff, off, blocks, tail):
     """Around the blocks of one and two passes of the whole grid (256 CUs x 8
     workgroups x 4 wavefronts), with partial last blocks and quads; blocks of
-    all byte values, data and output 16-byte aligned or 4 bytes past it."""
+    all byte values, data (doff) and output (off) 16-byte aligned or past it,
+    each by itself."""
     n = 256 * blocks + tail
     data = np.random.default_rng(blocks + t).integers(0, 256, blocks * TS[t], dtype=np.uint8)
-    db, dp = up(data, offset=off)
+    db, dp = up(data, offset=doff)
     ob = DeviceBuffer(4 * n + off + 16)
     ops.dequantize(t, dp, data.nbytes, n, ob.ptr + off)
     st, ref = orc.dequantize(t, data, n)
