@@ -225,8 +225,8 @@ def test_kquant_matmul_edges(gpu, orc, t, m, n, k):
 
 @pytest.mark.parametrize("t", [Q4_K, Q6_K])
 def test_kquant_nonfinite_scales(gpu, orc, t):
-    """A block scale d of inf or NaN makes its row NaN, as (d * s) * q does
-    where s or q is 0; the other rows are untouched."""
+    """A block scale d of inf (in a block with zero quants) or NaN makes its
+    row NaN, as (d * s) * q does where s or q is 0; the other rows are untouched."""
     m, n, k = 40, 96, 1024
     w = synth.quantized_weight(t, n, k, seed=5 + t).reshape(n, -1, TS[t]).copy()
     x = synth.activations(m * k, seed=6).reshape(m, k)
@@ -237,6 +237,58 @@ def test_kquant_nonfinite_scales(gpu, orc, t):
     got = kq_matmul(t, w.reshape(-1), x, m, n, k)
     assert np.all(np.isnan(got[:, [7, 50]]))
     rest = [r for r in range(n) if r not in (7, 50)]
+    assert np.array_equal(got[:, rest], base[:, rest])
+
+
+@pytest.mark.parametrize("t", [Q4_K, Q6_K])
+@pytest.mark.parametrize("m", [40, 130])
+def test_kquant_infinite_scales(gpu, orc, t, m):
+    """d of +-inf in a block without a zero scale or quant: the row is +-inf
+    where every product has one sign, as in the reference; NaN with one zero
+    quant or scale anywhere in the block, or with products of both signs."""
+    n, k = 96, 1024
+    w = synth.quantized_weight(t, n, k, seed=15 + t).reshape(n, -1, TS[t]).copy()
+    x = np.abs(synth.activations(m * k, seed=16)).reshape(m, k) + np.float32(0.01)
+    rng = np.random.default_rng(t)
+
+    def block(d):
+        if t == Q4_K:
+            return q4k_block(np.full(12, 0xFF, np.uint8), d, 0.5, rng.integers(1, 16, 128, dtype=np.uint8) * 17)
+        # no high bits: q - 32 is -32 .. -17 (the last element has no other choice)
+        return q6k_block(rng.integers(0, 256, 128, dtype=np.uint8), np.zeros(64, np.uint8),
+                         rng.integers(1, 256, 16, dtype=np.uint8), d)
+
+    rows = [3, 7, 20, 21, 22, 60, 95]
+    plain = w.copy()
+    for i, r in enumerate(rows):
+        b = block(-np.inf if r == 7 else np.inf)
+        if i == 2:                     # a zero quant (Q6_K: 32) among the first 64 elements
+            if t == Q4_K:
+                b[16] = 0x10
+            else:
+                b[0], b[128] = 0, 0x02
+        elif i == 3:                   # among the last 64 (Q6_K: element 250)
+            if t == Q4_K:
+                b[143] = 0x01
+            else:
+                b[122], b[190] = 0, 0x80
+        elif i == 4:                   # a zero scale
+            if t == Q4_K:
+                b[0] &= 0xC0
+            else:
+                b[207] = 0
+        elif i == 5:                   # 64 elements' products of the other sign
+            x[:, 768:832] *= -1
+        w[r, (0, 1, 2, 3, 0, 3, 2)[i]] = b
+    base = kq_matmul(t, plain.reshape(-1), x, m, n, k)
+    got = kq_matmul(t, w.reshape(-1), x, m, n, k)
+    for tok in (0, m - 1):
+        with np.errstate(all="ignore"):
+            ref = orc.matvec_f32(t, w.reshape(-1), x[tok], n, k)[1]
+        assert np.array_equal(np.isnan(got[tok]), np.isnan(ref))
+        inf = np.isinf(ref)
+        assert inf[[3, 7]].all() and np.array_equal(got[tok][inf], ref[inf])
+    rest = [r for r in range(n) if r not in rows]
     assert np.array_equal(got[:, rest], base[:, rest])
 
 

@@ -26,7 +26,6 @@ namespace {
 using whd::b16;
 using whd::kq_quad;
 using whd::q4k_scale;
-using whd::q6k_quant;
 
 template <int TYPE>
 constexpr int kq_bytes() { return TYPE == WH_TYPE_Q4_K ? 144 : 210; }
@@ -152,11 +151,15 @@ __global__ __launch_bounds__(256) void kq_gemv_kernel(const uint8_t* __restrict_
 // A K-quant matrix is rewritten once per handle or call into the stage records
 // of the prefill GEMM (kGemmQ4S, kGemmQ6S in wh_common.hpp): the integer
 // quants and sub-block scales as they are, the scales and d as floats.  d is
-// exact (times a power of two); one that is inf or NaN becomes NaN, since the
-// reference's d * s * q is NaN for it wherever s or q is 0.
-__device__ __forceinline__ float record_d(uint32_t bits16, float p) {
-  const float d = whd::f16_bits_to_f32(bits16);
-  return __builtin_fmaf(d, 0.f, d) * p;
+// exact (times a power of two).  An infinite d makes d * s * q infinite, or NaN
+// where s or q is 0; the GEMM multiplies d with sums of s * q * x, in which that
+// zero is lost, so the record's d is NaN then.  zero() tells whether any s or q
+// of the super-block is 0, and is asked for an infinite d only.
+template <typename Zero>
+__device__ __forceinline__ float record_d(uint32_t bits16, float p, Zero zero) {
+  float d = whd::f16_bits_to_f32(bits16) * p;
+  if ((bits16 & 0x7FFFu) == 0x7C00u && zero()) d = __builtin_nanf("");
+  return d;
 }
 
 // Q4_K: a workgroup stages one super-block of 64 rows in LDS (144-byte runs),
@@ -196,7 +199,17 @@ __global__ __launch_bounds__(256) void kq_repack_q4k_kernel(const uint8_t* __res
     rec[1] = make_uint2(split(qa.z), split(qa.w));
     rec[2] = make_uint2(split(qb.x), split(qb.y));
     rec[3] = make_uint2(split(qb.z), split(qb.w));
-    rec[4] = make_uint2(scale(pr & 63u) | (scale((pr >> 14) & 63u) << 16), __float_as_uint(record_d(h.w & 0xFFFFu, 16384.f)));
+    auto zero = [&]() {
+      const uint32_t* b = reinterpret_cast<const uint32_t*>(stage + 9 * row);
+      uint32_t z = 0;
+#pragma unroll 1
+      for (int i = 4; i < 36; i++) z |= (b[i] - 0x11111111u) & ~b[i] & 0x88888888u;  // a zero nibble
+#pragma unroll 1
+      for (int j = 0; j < 8; j++) z |= q4k_scale(reinterpret_cast<const uint8_t*>(b), j) == 0;
+      return z != 0;
+    };
+    rec[4] = make_uint2(scale(pr & 63u) | (scale((pr >> 14) & 63u) << 16),
+                        __float_as_uint(record_d(h.w & 0xFFFFu, 16384.f, zero)));
     if (s == 0) {
       uint16_t* tr = dmin_t + static_cast<size_t>(r0 + row) * dmin_stride;
       tr[sb] = static_cast<uint16_t>(h.w >> 16);
@@ -236,12 +249,11 @@ __global__ __launch_bounds__(256) void kq_repack_q6k_kernel(const uint8_t* __res
   }
   __syncthreads();
   const int s = wave, r = lane >> 1, half = lane & 1;
-  {
-    const uint32_t* b = stage + r * kQ6Stride;
-    const bool upper = s >= 2;
-    const int grp = 2 * s + half;               // elements 32 grp ..
-    uint32_t h[3] = {b[32 + 2 * grp], b[33 + 2 * grp], grp == 7 ? 0u : b[34 + 2 * grp]};
-    uint32_t q[8];
+  const uint32_t* b = stage + r * kQ6Stride;
+  // the quants of elements 32 grp .. 32 grp + 31, a byte each
+  auto quants = [&](int grp, uint32_t (&q)[8]) {
+    const bool upper = grp >= 4;
+    const uint32_t h[3] = {b[32 + 2 * grp], b[33 + 2 * grp], grp == 7 ? 0u : b[34 + 2 * grp]};
 #pragma unroll
     for (int c = 0; c < 8; c++) {
       const uint32_t nib = (b[4 * grp + (c & 3)] >> (upper ? 4 : 0)) & 0x0F0F0F0Fu;
@@ -249,17 +261,31 @@ __global__ __launch_bounds__(256) void kq_repack_q6k_kernel(const uint8_t* __res
       const uint32_t two = __builtin_amdgcn_alignbit(h[c / 4 + 1], h[c / 4], 8 * (c & 3)) >> (upper ? 2 : 0);
       q[c] = nib | (two & 3u) << 4 | (two & 0xCu) << 10 | (two & 0x30u) << 16 | (two & 0xC0u) << 22;
     }
-    uint4* rec = rec4[s] + 5 * r;
-    rec[2 * half] = make_uint4(q[0], q[1], q[2], q[3]);
-    rec[2 * half + 1] = make_uint4(q[4], q[5], q[6], q[7]);
-    const uint32_t sc = b[48 + s] >> (16 * half);  // scales 4s + 2 half, + 1
-    auto scale = [](uint32_t v) {
-      return static_cast<uint32_t>(__builtin_bit_cast(uint16_t, static_cast<_Float16>(static_cast<float>(v & 0xFFu))));
-    };
-    uint32_t* meta = reinterpret_cast<uint32_t*>(rec + 4);
-    meta[half] = scale(sc) | (scale(sc >> 8) << 16);
-    meta[2 + half] = half ? 0u : __float_as_uint(record_d(b[52] & 0xFFFFu, 0.015625f));
-  }
+  };
+  uint32_t q[8];
+  quants(2 * s + half, q);
+  uint4* rec = rec4[s] + 5 * r;
+  rec[2 * half] = make_uint4(q[0], q[1], q[2], q[3]);
+  rec[2 * half + 1] = make_uint4(q[4], q[5], q[6], q[7]);
+  const uint32_t sc = b[48 + s] >> (16 * half);  // scales 4s + 2 half, + 1
+  auto scale = [](uint32_t v) {
+    return static_cast<uint32_t>(__builtin_bit_cast(uint16_t, static_cast<_Float16>(static_cast<float>(v & 0xFFu))));
+  };
+  auto zero = [&]() {
+    auto zero_byte = [](uint32_t v) { return (v - 0x01010101u) & ~v & 0x80808080u; };
+    uint32_t z = zero_byte(b[48]) | zero_byte(b[49]) | zero_byte(b[50]) | zero_byte(b[51]);
+#pragma unroll 1
+    for (int grp = 0; grp < 8; grp++) {
+      uint32_t v[8];
+      quants(grp, v);
+#pragma unroll
+      for (int c = 0; c < 8; c++) z |= zero_byte(v[c] ^ 0x20202020u);  // q - 32
+    }
+    return z != 0;
+  };
+  uint32_t* meta = reinterpret_cast<uint32_t*>(rec + 4);
+  meta[half] = scale(sc) | (scale(sc >> 8) << 16);
+  meta[2 + half] = half ? 0u : __float_as_uint(record_d(b[52] & 0xFFFFu, 0.015625f, zero));
   __syncthreads();
   uint4* dst = reinterpret_cast<uint4*>(out + (static_cast<size_t>(4 * sb + s) * n_rows + r0) * 80);
   for (int i = lane; i < 5 * rows; i += 64) dst[i] = rec4[s][i];
