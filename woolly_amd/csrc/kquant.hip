@@ -162,18 +162,26 @@ __device__ __forceinline__ float record_d(uint32_t bits16, float p, Zero zero) {
   return d;
 }
 
+// Workgroup -> (row group, super-block), super-blocks fastest.  Consecutive
+// workgroups run on different XCDs, and a row's super-blocks share cache lines
+// (144 or 210 bytes each), so each XCD takes a contiguous part of the order
+// (Q4_K 14336 x 4096: 19.7 -> 16.9 us, 28672 x 8192: 65.6 -> 53.6 us).
+__device__ __forceinline__ unsigned kq_group() {
+  const unsigned q = gridDim.x / 8, rem = gridDim.x % 8, xcd = blockIdx.x % 8;
+  return xcd * q + min(xcd, rem) + blockIdx.x / 8;
+}
+
 // Q4_K: a workgroup stages one super-block of 64 rows in LDS (144-byte runs),
 // wave s forms their records of the super-block's stage s, and the records go
-// out through LDS as contiguous runs (read and written directly, 48 of 144 and
-// 8 of 40 bytes per lane and instruction, 14336 x 4096 took 17.1 us against
-// KQ4US).  16-byte aligned input.
+// out through LDS as contiguous runs.  16-byte aligned input.
 constexpr int kQ4Rows = 64;
 __global__ __launch_bounds__(256) void kq_repack_q4k_kernel(const uint8_t* __restrict__ w, int n_rows, unsigned nsb,
                                                             uint8_t* __restrict__ out, uint16_t* __restrict__ dmin_t,
                                                             int dmin_stride) {
   __shared__ uint4 stage[kQ4Rows * 9];
   __shared__ uint2 rec2[4][kQ4Rows * 5];
-  const int sb = static_cast<int>(blockIdx.x % nsb), r0 = static_cast<int>(blockIdx.x / nsb) * kQ4Rows;
+  const unsigned at = kq_group();
+  const int sb = static_cast<int>(at % nsb), r0 = static_cast<int>(at / nsb) * kQ4Rows;
   const int rows = min(kQ4Rows, n_rows - r0);
   const int s = static_cast<int>(threadIdx.x) >> 6, row = static_cast<int>(threadIdx.x) & 63;
   for (int i = threadIdx.x; i < 9 * rows; i += 256)
@@ -222,30 +230,37 @@ __global__ __launch_bounds__(256) void kq_repack_q4k_kernel(const uint8_t* __res
   for (int i = row; i < 5 * rows; i += 64) dst[i] = rec2[s][i];
 }
 
-// Q6_K: a workgroup stages one super-block of 32 rows in LDS (a wavefront per
-// row and load: the 210 bytes as dwords, which are only 2-byte aligned in
-// memory), each thread forms half a record: 32 elements share 16 bytes of ql
+// Q6_K: a workgroup stages one super-block of 32 rows in LDS (13 loads of 16
+// bytes and one of 2 per row, only 2-byte aligned in memory: 14336 x 4096 takes
+// 24.1 us with them, 35.3 with a dword per lane), each thread forms half a record: 32 elements share 16 bytes of ql
 // (element i and i + 16 the same byte) and 8 bytes of qh (9 for the upper half
 // of the block, whose bits start 2 higher and run into the next byte).  The
-// records go through LDS too, so that the stores are contiguous (80-byte
-// records stored as they are formed: 44 us for 14336 x 4096 against 35 us).
+// records go through LDS too, so that the stores are contiguous.
 constexpr int kQ6Rows = 32, kQ6Stride = 53;  // dwords per staged block
 __global__ __launch_bounds__(256) void kq_repack_q6k_kernel(const uint8_t* __restrict__ w, int n_rows, unsigned nsb,
                                                             uint8_t* __restrict__ out) {
   __shared__ uint32_t stage[kQ6Rows * kQ6Stride];
   __shared__ uint4 rec4[4][kQ6Rows * 5];
-  const int sb = static_cast<int>(blockIdx.x % nsb), r0 = static_cast<int>(blockIdx.x / nsb) * kQ6Rows;
+  const unsigned at = kq_group();
+  const int sb = static_cast<int>(at % nsb), r0 = static_cast<int>(at / nsb) * kQ6Rows;
   const int rows = min(kQ6Rows, n_rows - r0);
   const int wave = static_cast<int>(threadIdx.x) >> 6, lane = static_cast<int>(threadIdx.x) & 63;
 #pragma unroll
-  for (int i = 0; i < kQ6Rows / 4; i++) {
-    const int r = 4 * i + wave;
-    const uint8_t* b = w + (static_cast<size_t>(r0 + min(r, rows - 1)) * nsb + sb) * 210 + 4 * lane;
-    if (lane >= kQ6Stride) continue;
-    uint32_t v;
-    if (lane < kQ6Stride - 1) __builtin_memcpy(&v, b, 4);
-    else v = *reinterpret_cast<const uint16_t*>(b);  // the block's last two bytes: d
-    stage[r * kQ6Stride + lane] = v;
+  for (int i = 0; i < kQ6Rows * 14 / 256 + 1; i++) {
+    const int p = 256 * i + static_cast<int>(threadIdx.x), r = p / 14, c = p % 14;
+    if (r >= rows) break;
+    const uint8_t* b = w + (static_cast<size_t>(r0 + r) * nsb + sb) * 210 + 16 * c;
+    uint32_t* d = stage + r * kQ6Stride + 4 * c;
+    if (c < 13) {
+      uint4 v;
+      __builtin_memcpy(&v, b, 16);
+      d[0] = v.x;
+      d[1] = v.y;
+      d[2] = v.z;
+      d[3] = v.w;
+    } else {
+      d[0] = *reinterpret_cast<const uint16_t*>(b);  // the block's last two bytes: d
+    }
   }
   __syncthreads();
   const int s = wave, r = lane >> 1, half = lane & 1;
