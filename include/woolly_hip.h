@@ -252,7 +252,10 @@ WH_API int wh_swiglu(const float* gate, const float* up, size_t n, float* out,
  * (Q4_0, Q4_1, Q8_0, or Q4_K / Q6_K with hidden and n_ff multiples of 256).
  * The workspace must hold wh_ffn_workspace_bytes_for_type(type, hidden, n_ff, m)
  * bytes of device memory (no allocation happens inside the call);
- * wh_ffn_workspace_bytes(hidden, n_ff, m) is enough for Q4_0, Q4_1 and Q8_0. */
+ * wh_ffn_workspace_bytes(hidden, n_ff, m) is enough for Q4_0, Q4_1 and Q8_0.
+ * For Q4_K and Q6_K the size holds gate and up converted side by side where
+ * they run in one pass; one with room for one converted matrix at a time is
+ * taken too, and costs the one pass where both matrices need converting. */
 typedef struct wh_ffn_weights {
   int type;
   const void* gate;

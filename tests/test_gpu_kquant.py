@@ -9,7 +9,7 @@ import pytest
 from tests._gpu import down, gemv, up
 from tests._oracle import max_abs, rel_l2
 from tests.test_oracle_kquant import f16b, np_q4_k, np_q6_k, q4k_block, q6k_block
-from woolly_amd import gguf, ops, synth
+from woolly_amd import WoollyHipError, gguf, ops, synth
 from woolly_amd.device import DeviceBuffer
 
 pytestmark = pytest.mark.gpu
@@ -364,6 +364,50 @@ def test_kquant_ffn_parity(gpu, orc, t, hidden, n_ff, m):
     rms = float(np.sqrt(np.mean(ref ** 2)))
     print(f"[result] kquant ffn rel_l2={r:.3e} max_abs={a:.3e} rms={rms:.3e}", flush=True)
     assert r <= 1e-4 and a <= 1e-3 * max(1.0, rms / 300.0)
+
+
+@pytest.mark.parametrize("t", [Q4_K, Q6_K])
+@pytest.mark.parametrize("hidden,n_ff,m", [(4096, 14336, 130), (512, 20480, 257)])
+def test_kquant_ffn_workspace_sizes(gpu, orc, t, hidden, n_ff, m):
+    """Gate and up run in one pass here.  A workspace with room for one
+    converted matrix at a time is enough (unprepared matrices then run one after
+    the other where the scratch does not hold both); prepared handles give the
+    same bits in it as in the queried size; a byte less is refused."""
+    print(f"[case] kquant ffn workspace t={t} hidden={hidden} n_ff={n_ff} m={m}", flush=True)
+    up256 = lambda v: (v + 255) // 256 * 256
+    conv = lambda n, k: up256(n * (k // 32 * 20 + (k // 256 + 7) // 8 * 8 * 2) if t == Q4_K else n * k // 16 * 20)
+    rest = [ops.matmul_workspace_bytes(t, *nk, m) - conv(*nk) for nk in ((n_ff, hidden), (hidden, n_ff))]
+    least = up256(4 * m * hidden) + 3 * up256(4 * m * n_ff) + max(conv(n_ff, hidden), conv(hidden, n_ff)) + max(rest)
+    full = ops.ffn_workspace_bytes(hidden, n_ff, m, ggml_type=t)
+    # the query's extra: gate and up side by side, beyond the scratch that the one pass leaves
+    assert full == least + max(0, 2 * conv(n_ff, hidden) - 2 * up256(4 * m * n_ff) - max(conv(n_ff, hidden), conv(hidden, n_ff)))
+    L = synth.ffn_layer(t, hidden, n_ff, m, seed=hidden + n_ff + t)
+    bufs = {name: up(v) for name, v in L.items()}
+
+    def run(ptrs, wsz):
+        ob, ws = DeviceBuffer(4 * m * hidden), DeviceBuffer(wsz)
+        ops.ffn_swiglu(t, *ptrs, hidden, n_ff, bufs["gamma"][1], 1e-5, bufs["x"][1], m, ob.ptr, ws.ptr, wsz)
+        return down(ob, np.float32, m * hidden).reshape(m, hidden)
+
+    plain = [bufs[n][1] for n in ("gate", "up", "down")]
+    base = run(plain, full)
+    rows = sorted({0, m // 2, m - 1})
+    ref = orc.ffn_rows_f64(t, L["gate"], L["up"], L["down"], hidden, n_ff, L["gamma"], 1e-5, L["x"], rows)
+    for got in (base, run(plain, least)):
+        assert rel_l2(got[rows], ref) <= 4e-6   # two products behind each other, 2e-6 each as above
+    with pytest.raises(WoollyHipError) as e:
+        run(plain, least - 1)
+    assert e.value.status == 3
+    hw = [ops.Weight(t, *((n_ff, hidden) if n != "down" else (hidden, n_ff)), L[n]) for n in ("gate", "up", "down")]
+    for h in hw:
+        h.prepare_prefill()
+    for wsz in (full, least):
+        assert same(run([h.ptr for h in hw], wsz), base)
+    # one prepared, the other converted in the scratch
+    assert same(run([hw[0].ptr, plain[1], hw[2].ptr], full), base)
+    assert same(run([plain[0], hw[1].ptr, plain[2]], full), base)
+    for h in hw:
+        h.free()
 
 
 @pytest.mark.parametrize("t", [Q4_K, Q6_K])

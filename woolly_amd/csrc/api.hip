@@ -522,11 +522,13 @@ WH_API int wh_swiglu(const float* gate, const float* up, size_t n, float* out, w
 }
 
 // ------------------------------------------------------------------- FFN
-WH_API size_t wh_ffn_workspace_bytes_for_type(int type, size_t hidden, size_t n_ff, size_t m) {
+// least: the smallest that the call takes (a K-quant layer runs gate and up one
+// after the other in it where both need converting).
+static size_t ffn_workspace(int type, size_t hidden, size_t n_ff, size_t m, bool least) {
   size_t gemm_ws = 0;
   if (m > wh::kGemvTokenLimit) {
     if (wh::is_kquant(type)) {
-      gemm_ws = wh::ffn_kquant_workspace_bytes(type, hidden, n_ff, m);
+      gemm_ws = wh::ffn_kquant_workspace_bytes(type, hidden, n_ff, m, least);
     } else {
       const size_t g1 = wh::gemm_workspace_bytes_for(type, n_ff, m, hidden);
       const size_t g2 = wh::gemm_workspace_bytes_for(type, hidden, m, n_ff);
@@ -535,6 +537,10 @@ WH_API size_t wh_ffn_workspace_bytes_for_type(int type, size_t hidden, size_t n_
   }
   return align_up(m * hidden * sizeof(float), 256) + 3 * align_up(m * n_ff * sizeof(float), 256) +
          gemm_ws;
+}
+
+WH_API size_t wh_ffn_workspace_bytes_for_type(int type, size_t hidden, size_t n_ff, size_t m) {
+  return ffn_workspace(type, hidden, n_ff, m, false);
 }
 
 // Enough for each of Q4_0, Q4_1 and Q8_0.
@@ -556,7 +562,7 @@ WH_API int wh_ffn_swiglu(const wh_ffn_weights* w, const float* gamma, float eps,
   st = check_gemv_args("ffn_swiglu", w->type, w->n_ff);
   if (st) return st;
   if (m == 0 || w->hidden == 0) return WH_OK;
-  const size_t need = wh_ffn_workspace_bytes_for_type(w->type, w->hidden, w->n_ff, m);
+  const size_t need = ffn_workspace(w->type, w->hidden, w->n_ff, m, true);
   if (workspace_bytes < need)
     return wh::set_error(WH_ERR_BUFFER_TOO_SMALL,
                          "ffn_swiglu: workspace too small: needed %zu bytes, available %zu", need,
@@ -578,7 +584,7 @@ WH_API int wh_ffn_swiglu(const wh_ffn_weights* w, const float* gamma, float eps,
   float* h = reinterpret_cast<float*>(ws);
   ws += align_up(m * F * sizeof(float), 256);
   void* gemm_ws = ws;
-  const size_t gemm_bytes = need - static_cast<size_t>(ws - static_cast<char*>(workspace));
+  const size_t gemm_bytes = workspace_bytes - static_cast<size_t>(ws - static_cast<char*>(workspace));
   hipStream_t s = hs(stream);
   if (F == 0) return wh::launch_fill_bytes(out, 0, m * H * sizeof(float), s);
   if (m >= 2 && m <= 16 && wh::mt_allowed(F, H)) {

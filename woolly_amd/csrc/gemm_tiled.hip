@@ -1244,35 +1244,44 @@ static bool ffn_one_pass(int it, size_t n_ff, size_t n_tokens, size_t hidden) {
   return gemm_tiled_splits(it, 2 * n_ff, n_tokens, hidden) == 1;
 }
 
-// Gate and up in one pass need both matrices repacked at the same time.
-size_t ffn_kquant_workspace_bytes(int type, size_t hidden, size_t n_ff, size_t n_tokens) {
+// Room for the repacked matrices.  The least is one at a time; gate and up in
+// one pass need both, and use the scratch of the outputs that pass does not
+// write too (u and h, launch_ffn_tiled).
+static size_t ffn_repacked_bytes(int type, size_t hidden, size_t n_ff, size_t n_tokens, bool least) {
+  const size_t r1 = al256(kquant_repacked_bytes(type, n_ff, hidden)), r2 = al256(kquant_repacked_bytes(type, hidden, n_ff));
+  size_t b = r1 > r2 ? r1 : r2;
+  if (!least && ffn_one_pass(kquant_gemm_type(type), n_ff, n_tokens, hidden)) {
+    const size_t scratch = 2 * al256(n_tokens * n_ff * 4);
+    if (2 * r1 > scratch + b) b = 2 * r1 - scratch;
+  }
+  return b;
+}
+
+size_t ffn_kquant_workspace_bytes(int type, size_t hidden, size_t n_ff, size_t n_tokens, bool least) {
   const int it = kquant_gemm_type(type);
-  const size_t r1 = al256(kquant_repacked_bytes(type, n_ff, hidden)) * (ffn_one_pass(it, n_ff, n_tokens, hidden) ? 2 : 1);
-  const size_t r2 = al256(kquant_repacked_bytes(type, hidden, n_ff));
   const size_t t1 = gemm_tiled_workspace_bytes(it, n_ff, n_tokens, hidden);
   const size_t t2 = gemm_tiled_workspace_bytes(it, hidden, n_tokens, n_ff);
-  return (r1 > r2 ? r1 : r2) + (t1 > t2 ? t1 : t2);
+  return ffn_repacked_bytes(type, hidden, n_ff, n_tokens, least) + (t1 > t2 ? t1 : t2);
 }
 
 // The FFN for n_tokens rows on the tiled kernel: the RMSNorm of x is packed
 // once for both gate and up, the SwiGLU of their outputs is formed while the
-// down projection's activations are packed.  g, u: n_tokens x n_ff scratch.
+// down projection's activations are packed.  g, u: n_tokens x n_ff scratch; u
+// and all between it and the workspace, which follows, may be overwritten.
 // WH_ERR_INVALID_SHAPE (nothing launched) when a product does not fit.
 int launch_ffn_tiled(int type, const void* gate, const void* up, const void* down, size_t hidden, size_t n_ff,
                      const float* x, const float* gamma, float eps, size_t n_tokens, float* g, float* u, float* out,
                      void* workspace, size_t workspace_bytes, hipStream_t s) {
   if (is_kquant(type)) {
-    // the repacked matrices in the front of the workspace: gate and up side by
-    // side for one pass, else one at a time (stream order keeps a GEMM's reads
-    // ahead of the next repack)
+    // the repacked matrices in the front of the workspace (stream order keeps a
+    // GEMM's reads ahead of the next repack)
     const int it = kquant_gemm_type(type);
-    const bool one = ffn_one_pass(it, n_ff, n_tokens, hidden);
-    const size_t r1 = al256(kquant_repacked_bytes(type, n_ff, hidden)), r2 = al256(kquant_repacked_bytes(type, hidden, n_ff));
+    const bool full = workspace_bytes >= ffn_kquant_workspace_bytes(type, hidden, n_ff, n_tokens, false);
     char* rp = static_cast<char*>(workspace);
-    char* ws = rp + (r1 * (one ? 2 : 1) > r2 ? r1 * (one ? 2 : 1) : r2);
+    char* ws = rp + ffn_repacked_bytes(type, hidden, n_ff, n_tokens, !full);
     if (!gemm_kquant_ok(type, gate, x, n_ff, hidden, n_tokens) || !aligned(up, 16) || !aligned(down, 16) ||
         !gemm_kquant_ok(type, down, g, hidden, n_ff, n_tokens) || !aligned(gamma, 16) || !aligned(u, 16) ||
-        !aligned(workspace, 256) || workspace_bytes < ffn_kquant_workspace_bytes(type, hidden, n_ff, n_tokens))
+        !aligned(workspace, 256) || workspace_bytes < ffn_kquant_workspace_bytes(type, hidden, n_ff, n_tokens, true))
       return WH_ERR_INVALID_SHAPE;
     // each matrix: its handle's prepared copy, or converted into `at` for this call
     auto repacked = [&](const void* w, size_t rows, size_t k, char* at, const char** out_rp) -> int {
@@ -1280,14 +1289,22 @@ int launch_ffn_tiled(int type, const void* gate, const void* up, const void* dow
       *out_rp = pre ? pre : at;
       return pre ? WH_OK : launch_repack_kquant(type, w, rows, k, at, s);
     };
+    // gate and up in one pass: those that need converting go side by side into
+    // [u, ws), which that pass does not use; in a smaller workspace, where they
+    // do not fit, one after the other
+    char* both = reinterpret_cast<char*>(al256(reinterpret_cast<size_t>(u)));
+    const size_t r1 = al256(kquant_repacked_bytes(type, n_ff, hidden));
+    const size_t gate_bytes = prepared_kquant(gate, type, n_ff, hidden) ? 0 : r1;
+    const size_t up_bytes = prepared_kquant(up, type, n_ff, hidden) ? 0 : r1;
+    const bool one = ffn_one_pass(it, n_ff, n_tokens, hidden) && gate_bytes + up_bytes <= static_cast<size_t>(ws - both);
     const char *src = nullptr, *src2 = nullptr;
     const TiledWs t1 = tiled_ws(it, n_ff, hidden, n_tokens, ws);
     const TiledWs t2 = tiled_ws(it, hidden, n_ff, n_tokens, ws);
     int st = tiled_pack<kPackNorm>(it, t1, x, nullptr, gamma, eps, n_tokens, hidden, s);
-    if (!st) st = repacked(gate, n_ff, hidden, rp, &src);
+    if (!st) st = repacked(gate, n_ff, hidden, one ? both : rp, &src);
     if (one) {
       // h = silu(g) * u written by the epilogue (g holds h)
-      if (!st) st = repacked(up, n_ff, hidden, rp + r1, &src2);
+      if (!st) st = repacked(up, n_ff, hidden, both + gate_bytes, &src2);
       if (!st) st = sb_run(it, reinterpret_cast<const uint8_t*>(src), reinterpret_cast<const uint8_t*>(src2), n_ff, hidden,
                            n_tokens, t1, g, 1, 0, true, s);
       if (!st) st = tiled_pack<kPackPlain>(it, t2, g, nullptr, nullptr, 0.f, n_tokens, n_ff, s);

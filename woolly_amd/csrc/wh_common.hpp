@@ -195,11 +195,14 @@ bool gemm_kquant_ok(int type, const void* w, const float* x, size_t n_rows, size
 size_t gemm_kquant_workspace_bytes(int type, size_t n_rows, size_t n_tokens, size_t k);
 int launch_gemm_kquant(int type, const void* w, size_t n_rows, size_t k, const float* x, size_t n_tokens,
                        float* y, void* workspace, hipStream_t stream, bool xb = false);
-// Workspace of launch_ffn_tiled beyond its g / u scratch, for a K-quant FFN.
-size_t ffn_kquant_workspace_bytes(int type, size_t hidden, size_t n_ff, size_t n_tokens);
+// Workspace of launch_ffn_tiled beyond its g / u scratch, for a K-quant FFN; the
+// least that it takes (one converted matrix at a time), or with room for gate
+// and up side by side.
+size_t ffn_kquant_workspace_bytes(int type, size_t hidden, size_t n_ff, size_t n_tokens, bool least);
 // FFN for more than kGemvTokenLimit tokens on the tiled kernel, with the
 // RMSNorm and SwiGLU fused into its activation packing (g, u: scratch of
-// n_tokens x n_ff); WH_ERR_INVALID_SHAPE (nothing launched) when it does not fit.
+// n_tokens x n_ff; u and all from it up to the workspace, which lies behind it
+// in one buffer, may be overwritten); WH_ERR_INVALID_SHAPE (nothing launched) when it does not fit.
 int launch_ffn_tiled(int type, const void* gate, const void* up, const void* down, size_t hidden, size_t n_ff,
                      const float* x, const float* gamma, float eps, size_t n_tokens, float* g, float* u, float* out,
                      void* workspace, size_t workspace_bytes, hipStream_t s);
