@@ -213,3 +213,17 @@ def test_embedding_lookup_argument_errors_need_no_gpu():
     from woolly_amd import ops
     with pytest.raises(ValueError, match="Token ID 10 exceeds vocabulary size 10"):
         ops.embedding_lookup(2, 0x10000, 10, 256, [3, 10], 0x10000)
+
+
+@pytest.mark.parametrize("t", [12, 14])
+@pytest.mark.parametrize("nsb,planes", [(16, 16), (17, 9), (20, 10), (33, 11), (36, 12), (56, 14)])
+def test_kquant_split_k_has_no_empty_planes(t, nsb, planes):
+    """10 tiles of 256 rows at 20 tokens: up to 16 K-splits of whole
+    super-blocks; the workspace holds a plane per split that has any."""
+    lib = _lib.load()
+    up = lambda v: (v + 255) // 256 * 256
+    n, k, m, tm = 2560, 256 * nsb, 20, 32
+    conv = n * (k // 64 * 40 + (nsb + 7) // 8 * 16 if t == 12 else k // 64 * 80)
+    sums = up(tm * ((nsb + 7) // 8 * 8) * 4) if t == 12 else 0
+    assert lib.wh_quantized_matmul_workspace_bytes(t, n, k, m) == \
+        up(conv) + up(tm * k * 4) + up(tm * 4) + sums + up(planes * n * m * 4)

@@ -1023,7 +1023,8 @@ bool gemm_tiled_ok(int type, const void* w, const float* x, size_t n_rows, size_
 
 // Split-K factor: the largest power of two up to 8 that keeps the workgroups
 // within one per CU and every split at least 16 blocks deep (the K-quant
-// kernel: 16, and one super-block).
+// kernel: 16, and one super-block; planes that whole super-blocks per split
+// would leave empty are not formed: 17 super-blocks in 16 splits are 9 of two).
 int gemm_tiled_splits(int type, size_t n_rows, size_t n_tokens, size_t k) {
   const size_t bm = static_cast<size_t>(tile_bm(type, n_tokens));
   const size_t tiles = ((n_rows + TBN - 1) / TBN) * ((n_tokens + bm - 1) / bm);
@@ -1031,8 +1032,10 @@ int gemm_tiled_splits(int type, size_t n_rows, size_t n_tokens, size_t k) {
   const size_t cus = static_cast<size_t>(cu_count());
   int s = 1;
   if (is_sb(type)) {  // whole super-blocks, down to one per split
-    while (s < 16 && tiles * s * 2 <= cus && k / 256 >= static_cast<size_t>(2 * s)) s *= 2;
-    return s;
+    const size_t nsb = k / 256;
+    while (s < 16 && tiles * s * 2 <= cus && nsb >= static_cast<size_t>(2 * s)) s *= 2;
+    const size_t per = (nsb + s - 1) / s;
+    return static_cast<int>((nsb + per - 1) / per);
   }
   while (s < 8 && tiles * s * 2 <= cus && nb / (2 * s) >= 16) s *= 2;
   return s;
