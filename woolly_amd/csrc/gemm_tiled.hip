@@ -856,14 +856,33 @@ int tile_bm(int type, size_t n_tokens) {
 // CU whenever the tiles do not fill the CUs evenly (a last round with idle
 // CUs, or fewer tiles than CUs, where split-K planes and a reduce would
 // otherwise be needed) and every workgroup's share is at least 8 stages; 0
-// (one workgroup per tile) otherwise.  Every block format of the kernel.
-// (The K-quant kernel's units are super-blocks of four stages.)
-int sk_grid(int type, size_t n_tiles, size_t tile_st) {
+// (one workgroup per tile and split) otherwise.  The 32-element formats.
+int sk_grid(size_t n_tiles, size_t tile_st) {
   const size_t g = static_cast<size_t>(wh::cu_count());
   if (g == 0 || g % 8 != 0 || n_tiles % g == 0) return 0;
-  if (is_sb(type)) return (n_tiles * (tile_st / 4) + g - 1) / g >= 2 ? static_cast<int>(g) : 0;
   const size_t upw = (n_tiles * tile_st + g - 1) / g;
   return upw >= 8 ? static_cast<int>(g) : 0;
+}
+
+// The same for the K-quant kernel, whose units are super-blocks (nsb per tile;
+// bm: tokens per tile; splits: what split-K would take).  A tile's owners hand
+// their parts over one after the other, so with more than four, stream-K loses
+// to split-K planes and a reduce (100 tokens, Q4_K, stream-K / split-K in us:
+// 5 tiles of 56 super-blocks 77.3 / 53.4, 16 of 32 56.0 / 42.4, 32 of 22 54.4 /
+// 47.1, 32 of 56 85.2 / 81.1).  With up to four it wins where it shortens the
+// longest workgroup by more than an eighth (40 of 22, four super-blocks instead
+// of six: 56.1 / 62.9; 80 of 16, five of eight: 64.8 / 73.3), and not below that
+// (56 of 32, seven of eight: 84.2 / 77.4; 64 of 22, six of six: 73.9 / 69.5).
+// 64-token tiles hand over half as much: they gain with up to four in any case
+// (60 tokens, 64 of 8: 27.0 / 28.8; 64 of 22 47.1 / 45.6).  Without split-K it
+// needs any shortening.
+int sb_sk_grid(size_t n_tiles, size_t nsb, int bm, int splits) {
+  const size_t g = static_cast<size_t>(wh::cu_count());
+  if (g == 0 || g % 8 != 0 || n_tiles % g == 0 || bm < 64 || splits > 4) return 0;
+  const size_t upw = (n_tiles * nsb + g - 1) / g;
+  const size_t per = (n_tiles * splits + g - 1) / g * ((nsb + splits - 1) / splits);
+  const bool gain = splits == 1 ? upw < per : bm == 64 || 8 * upw < 7 * per;
+  return upw >= 2 && gain ? static_cast<int>(g) : 0;
 }
 
 // The stream-K state of a launch: flags and partial slots (SkWs::g workgroups).
@@ -888,7 +907,7 @@ int launch_bm_lo(const uint8_t* w, size_t n_rows, size_t k, size_t n_tokens, con
   const int n_tiles = tiles_m * tiles_n;
   const size_t lds = tiled_lds_bytes<TYPE, BM>();
   {
-    if (splits == 1 && sk.g > 0 && sk_grid(TYPE, n_tiles, nb / SB) == sk.g) {
+    if (splits == 1 && sk.g > 0 && sk_grid(n_tiles, nb / SB) == sk.g) {
       const int upw = (n_tiles * (nb / SB) + sk.g - 1) / sk.g;
       WH_ENSURE_LDS(lds, &gemm_tiled_kernel<TYPE, BM, false, true, LO>);
       gemm_tiled_kernel<TYPE, BM, false, true, LO><<<static_cast<unsigned>(sk.g), TWAVES * 64, lds, s>>>(
@@ -931,7 +950,7 @@ int launch_ffn_bm(const uint8_t* gate, const uint8_t* up, size_t n_ff, size_t k,
   const int tiles_m = static_cast<int>((n_tokens + BM - 1) / BM);
   const int n_tiles = tiles_m * tiles_n;
   const size_t lds = tiled_lds_bytes<TYPE, BM>();
-  if (sk.g > 0 && sk_grid(TYPE, n_tiles, nb / SB) == sk.g) {
+  if (sk.g > 0 && sk_grid(n_tiles, nb / SB) == sk.g) {
     const int upw = (n_tiles * (nb / SB) + sk.g - 1) / sk.g;
     WH_ENSURE_LDS(lds, &gemm_tiled_kernel<TYPE, BM, true, true>);
     gemm_tiled_kernel<TYPE, BM, true, true><<<static_cast<unsigned>(sk.g), TWAVES * 64, lds, s>>>(
@@ -1049,8 +1068,9 @@ int gemm_tiled_splits(int type, size_t n_rows, size_t n_tokens, size_t k) {
 // 14336 x 4096: 31.9 against 31.3 us).
 static int sk_plain(int type, size_t n_rows, size_t n_tokens, size_t k) {
   const size_t bm = static_cast<size_t>(tile_bm(type, n_tokens));
-  if (bm < 64) return 0;
-  return sk_grid(type, ((n_tokens + bm - 1) / bm) * ((n_rows + TBN - 1) / TBN), k / 32 / SB);
+  const size_t tiles = ((n_tokens + bm - 1) / bm) * ((n_rows + TBN - 1) / TBN);
+  if (is_sb(type)) return sb_sk_grid(tiles, k / 256, static_cast<int>(bm), gemm_tiled_splits(type, n_rows, n_tokens, k));
+  return bm < 64 ? 0 : sk_grid(tiles, k / 32 / SB);
 }
 // Split-K factor of the GEMM over n_rows rows: 1 where it runs stream-K.
 static int tiled_splits(int type, size_t n_rows, size_t n_tokens, size_t k) {
@@ -1061,7 +1081,8 @@ static int sk_slots(int type, size_t n_rows, size_t n_tokens, size_t k) {
   if (g) return g;
   if (gemm_tiled_splits(type, 2 * n_rows, n_tokens, k) == 1 && tile_bm(type, n_tokens) >= 64) {
     const size_t bm = static_cast<size_t>(tile_bm(type, n_tokens));
-    return sk_grid(type, ((n_tokens + bm - 1) / bm) * ((n_rows + TBN / 2 - 1) / (TBN / 2)), k / 32 / SB);
+    const size_t tiles = ((n_tokens + bm - 1) / bm) * ((n_rows + TBN / 2 - 1) / (TBN / 2));
+    return is_sb(type) ? sb_sk_grid(tiles, k / 256, static_cast<int>(bm), 1) : sk_grid(tiles, k / 32 / SB);
   }
   return 0;
 }
@@ -1152,9 +1173,10 @@ static int sb_run(int type, const uint8_t* w, const uint8_t* w2, size_t n_rows, 
   a.splits = splits;
   a.ffn = w2 != nullptr;
   a.lo = lo;
-  const size_t tn = w2 ? TBN / 2 : TBN;
-  const size_t tiles = (n_rows + tn - 1) / tn * (t.tm / t.bm);
-  if (splits == 1 && t.sk_n > 0 && sk_grid(type, tiles, k / 64) == t.sk_n) {
+  // stream-K: the FFN's one pass by its own tiles, else as sk_plain laid it out
+  const int sk = w2 ? sb_sk_grid((n_rows + TBN / 2 - 1) / (TBN / 2) * (t.tm / t.bm), k / 256, t.bm, 1)
+                    : sk_plain(type, n_rows, n_tokens, k);
+  if (sk > 0 && sk == t.sk_n) {
     a.sk_flags = t.sk_flags;
     a.sk_part = t.sk_part;
     a.sk_g = t.sk_n;
