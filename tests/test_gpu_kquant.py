@@ -223,6 +223,26 @@ def test_kquant_matmul_edges(gpu, orc, t, m, n, k):
     assert np.array_equal(down(yb, np.float32, m * n).reshape(m, n), got)
 
 
+# one to three super-blocks per workgroup, in tiles of 32, 64 and (Q4_K) 128 tokens
+KQ_SHORT = [(20, 2048, 1024), (50, 1024, 2048), (64, 2048, 1024), (100, 2048, 1024), (150, 3000, 2816), (130, 4096, 1280)]
+
+
+@pytest.mark.parametrize("t", [Q4_K, Q6_K])
+@pytest.mark.parametrize("m,n,k", KQ_SHORT)
+def test_kquant_short_sums(gpu, orc, t, m, n, k):
+    """Short sums hide no rounding.  In units of one f32 rounding of a normal
+    variate (2.53e-8 rms, relative): the 22-bit activations add 5.6, the f32
+    sum of a super-block's four chains 2.2, the planes' 1, and the matrix cores,
+    which round four times per product at the size of the chain, 4.8 to 5.4 (5.4
+    and x_lo w_lo left out 0.8): sqrt(15) = 0.98e-7.  Two products of lo limbs
+    between the x_hi w_hi of a chain's steps make that 8.5: 1.08e-7."""
+    w = synth.quantized_weight(t, n, k, seed=n + k + t)
+    x = synth.activations(m * k, seed=m + t).reshape(m, k)
+    r = rel_l2(kq_matmul(t, w, x, m, n, k), orc.matmul_rows_f64(t, w, n, k, x, m, np.arange(m)))
+    print(f"[result] kquant short sums t={t} m={m} n={n} k={k} rel_l2={r:.3e}", flush=True)
+    assert r <= 1.05e-7
+
+
 @pytest.mark.parametrize("t", [Q4_K, Q6_K])
 def test_kquant_nonfinite_scales(gpu, orc, t):
     """A block scale d of inf (in a block with zero quants) or NaN makes its

@@ -66,6 +66,24 @@ constexpr int sb_rec() { return TYPE == wh::kGemmQ4S ? 40 : 80; }  // bytes per 
 // us with 64, 120.6 with 128; at M=128 55.1 and 53.5.
 inline int sb_chain(int bm, int sb) { return bm == 128 && sb >= 8 ? 1 : 0; }
 
+// Q6_K where a workgroup sums one or two super-blocks: the products with an x_lo
+// or w_lo of both steps of a stage come before the x_hi w_hi of either (1).  An
+// MFMA rounds four times at the size of C, and the two products of lo limbs
+// between the x_hi w_hi of the two steps are most of a short sum's error.
+// 2: x_lo w_lo too, in the 64-token tiles of a longer prompt (gemm_tiled.hip's
+// tile_bm: up to four super-blocks).  Error against 64
+// bits (with 0; with one scale per 16 elements, whose quants are exact), 1e-7:
+// 2048 x 1024 at 20 and 64 tokens 0.93 (1.07; 0.98), at 100 0.86 (1.08; 1.00),
+// 1024 x 2048 at 50 0.97 (1.18; 1.08), 4096 x 4096 at 20 1.02 (1.34; 1.32).  Time
+// 2048 x 1024 at 20 tokens 14.0 us (13.7), 14336 x 1024 at 64 26.6 us (26.1); the
+// longer sums of 14336 x 4096 do not need it (1.29; 1.59) and would take 29.3 us
+// instead of 28.2 at 32 tokens.
+inline int sb_lo_first(int type, int bm, int n_tokens, int sb, bool ffn) {
+  if (type != wh::kGemmQ6S || bm > 64 || ffn) return 0;
+  if (n_tokens > 64) return 2;
+  return sb <= 2 ? 1 : 0;
+}
+
 template <int TYPE, int BM, bool LO>
 struct SbStage {
   static constexpr int FR = BM / 16 * (LO ? 2 : 1);              // fragments per step
@@ -92,7 +110,7 @@ __device__ __forceinline__ half2v sb_nib(uint32_t u, uint32_t mask, half2v s) {
 
 // Weight rows r0.. of one tile, K stages [st_a, st_b): the GEMM over it.  Grid
 // and stream-K (SK) as gemm_tiled_kernel; units are super-blocks.
-template <int TYPE, int BM, bool FFNP, bool SK, bool LO>
+template <int TYPE, int BM, bool FFNP, bool SK, bool LO, int LF>
 __global__ __launch_bounds__(TWAVES * 64, 1) void gemm_sb_kernel(
     const uint8_t* __restrict__ W, const uint8_t* __restrict__ W2, const _Float16* __restrict__ frag,
     const float* __restrict__ rscale, const float* __restrict__ bsum, float* __restrict__ y, int n_tokens, int n_rows,
@@ -200,6 +218,7 @@ __global__ __launch_bounds__(TWAVES * 64, 1) void gemm_sb_kernel(
   const uint32_t d_lds = w_lds + (Q4 ? 36 - 8 * g : 72 - 16 * g);
 
   half8 ah[IT], al[IT], bw[NT], bl[NT];
+  half8 ah1[IT], al1[IT], bw1[NT];  // LF: the stage's second step
   uint2 rq[NT];          // quants: Q4_K both steps of the stage, Q6_K one step
   half2v sc[NT];         // the lane's scale of the stage in both halves
   float dn[NT];          // d of the chain whose products are pending
@@ -225,6 +244,12 @@ __global__ __launch_bounds__(TWAVES * 64, 1) void gemm_sb_kernel(
       sc[n] = half2v{sv, sv};
     }
   };
+  // Q6_K: pair c of q - 32: bytes under 0x64 are fp16 1024 + q; minus 1056
+  auto q6_pair = [](uint2 q, int c) {
+    const half2v off = {static_cast<_Float16>(-1056.f), static_cast<_Float16>(-1056.f)};
+    const uint32_t w = __builtin_amdgcn_perm(0x64646464u, c < 2 ? q.x : q.y, (c & 1) ? 0x04030402u : 0x04010400u);
+    return __builtin_bit_cast(half2v, w) + off;
+  };
   // weights of row group n for step t from rq / sc
   auto form = [&](int n, int t) {
     half2v p[4];
@@ -236,13 +261,8 @@ __global__ __launch_bounds__(TWAVES * 64, 1) void gemm_sb_kernel(
       p[2] = sb_nib(q >> 8, 0x000F000Fu, sc[n]);
       p[3] = sb_nib(q >> 8, 0x00F000F0u, s16);
     } else {
-      const half2v off = {static_cast<_Float16>(-1056.f), static_cast<_Float16>(-1056.f)};
 #pragma unroll
-      for (int c = 0; c < 4; c++) {
-        // bytes under 0x64: fp16 1024 + q; minus 1056: q - 32; times s, rounded
-        const uint32_t w = __builtin_amdgcn_perm(0x64646464u, c < 2 ? rq[n].x : rq[n].y, (c & 1) ? 0x04030402u : 0x04010400u);
-        p[c] = (__builtin_bit_cast(half2v, w) + off) * sc[n];
-      }
+      for (int c = 0; c < 4; c++) p[c] = q6_pair(rq[n], c) * sc[n];  // rounded
     }
 #pragma unroll
     for (int c = 0; c < 4; c++) {
@@ -252,12 +272,10 @@ __global__ __launch_bounds__(TWAVES * 64, 1) void gemm_sb_kernel(
   };
   // Q6_K: the rest s (q - 32) - hi of row group n
   auto form_lo = [&](int n) {
-    const half2v off = {static_cast<_Float16>(-1056.f), static_cast<_Float16>(-1056.f)};
 #pragma unroll
     for (int c = 0; c < 4; c++) {
-      const uint32_t w = __builtin_amdgcn_perm(0x64646464u, c < 2 ? rq[n].x : rq[n].y, (c & 1) ? 0x04030402u : 0x04010400u);
       const half2v hi = {bw[n][2 * c], bw[n][2 * c + 1]};
-      const half2v r = __builtin_elementwise_fma(__builtin_bit_cast(half2v, w) + off, sc[n], -hi);
+      const half2v r = __builtin_elementwise_fma(q6_pair(rq[n], c), sc[n], -hi);
       bl[n][2 * c] = r[0];
       bl[n][2 * c + 1] = r[1];
     }
@@ -312,7 +330,7 @@ __global__ __launch_bounds__(TWAVES * 64, 1) void gemm_sb_kernel(
   } else {
     if constexpr (LO) read_a(smem, 0, 1, al);
 #pragma unroll
-    for (int n = 0; n < NT / 2; n++) form(n, 0);
+    for (int n = 0; n < (LF ? NT : NT / 2); n++) form(n, 0);
   }
   int cur = 0;  // slot of the stage computed
   // One stage per trip: unrolled over the four of a super-block the body
@@ -334,6 +352,74 @@ __global__ __launch_bounds__(TWAVES * 64, 1) void gemm_sb_kernel(
         asm volatile("" ::: "memory");
         issue();
       };
+      if constexpr (LF != 0) {
+        auto step = [&](half8 (&a)[IT], half8 (&b)[NT], auto then) {
+#pragma unroll
+          for (int n = 0; n < NT; n++) {
+#pragma unroll
+            for (int i = 0; i < IT; i++) mma(i, n, a[i], b[n]);
+            then(n);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+        };
+        uint2 rq1[NT];
+        // the first step's x_lo w_hi; its x_hi and the second's x_lo and quants read
+        read_a(slot, 0, 0, ah);
+        if constexpr (LO) read_a(slot, 1, 1, al1);
+#pragma unroll
+        for (int n = 0; n < NT; n++) rq1[n] = *reinterpret_cast<const uint2*>(slot + w_lds + w_grp(n) + 8);
+#pragma unroll
+        for (int n = 0; n < NT; n++) {
+#pragma unroll
+          for (int i = 0; i < IT; i++)
+            if constexpr (LO) mma(i, n, al[i], bw[n]);
+          if (head && n == 0) apply(NT - 1, dn[NT - 1]);
+          form_lo(n);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        // its x_hi w_lo; the second step's weights formed and its x_hi read
+        read_a(slot, 1, 0, ah1);
+        if (tail) read_d(slot);
+        if constexpr (LO && LF == 2) step(al, bl, [](int) {});
+        step(ah, bl, [&](int n) {
+          rq[n] = rq1[n];
+#pragma unroll
+          for (int c = 0; c < 4; c++) {
+            const half2v p = q6_pair(rq1[n], c) * sc[n];
+            bw1[n][2 * c] = p[0];
+            bw1[n][2 * c + 1] = p[1];
+          }
+        });
+        // the second step's x_lo w_hi
+#pragma unroll
+        for (int n = 0; n < NT; n++) {
+#pragma unroll
+          for (int i = 0; i < IT; i++)
+            if constexpr (LO) mma(i, n, al1[i], bw1[n]);
+#pragma unroll
+          for (int c = 0; c < 4; c++) {
+            const half2v hi = {bw1[n][2 * c], bw1[n][2 * c + 1]};
+            const half2v r = __builtin_elementwise_fma(q6_pair(rq[n], c), sc[n], -hi);
+            bl[n][2 * c] = r[0];
+            bl[n][2 * c + 1] = r[1];
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        turn();
+        read_q(nslot, 0);
+        read_s(nslot);
+        if constexpr (LO && LF == 2) step(al1, bl, [](int) {});
+        step(ah1, bl, [](int) {});
+        // x_hi w_hi of both; the next stage's x_lo read and weights formed
+        if constexpr (LO) read_a(nslot, 0, 1, al);
+        step(ah, bw, [](int) {});
+        step(ah1, bw1, [&](int n) {
+          if (tail && n > 0) apply(n - 1, dn[n - 1]);
+          form(n, 0);
+        });
+        cur = nxt;
+        continue;
+      }
 #pragma unroll
       for (int t = 0; t < 2; t++) {
         const bool zero = head && t == 0, last = tail && t == 1;
@@ -563,17 +649,18 @@ __global__ __launch_bounds__(TWAVES * 64, 1) void gemm_sb_kernel(
   }  // segment
 }
 
-template <int TYPE, int BM, bool FFNP, bool SK, bool LO>
+template <int TYPE, int BM, bool FFNP, bool SK, bool LO, int LF = 0>
 int sb_launch(const wh::SbGemm& a, hipStream_t s) {
   const int tiles_n = (a.n_rows + (FFNP ? TBN / 2 : TBN) - 1) / (FFNP ? TBN / 2 : TBN);
   const int n_tiles = (a.n_tokens + BM - 1) / BM * tiles_n;
   const int nsb = a.k / 256;
   const size_t lds = static_cast<size_t>(SbStage<TYPE, BM, LO>::N) * SbStage<TYPE, BM, LO>::BYTES;
-  WH_ENSURE_LDS(lds, &gemm_sb_kernel<TYPE, BM, FFNP, SK, LO>);
+  auto* kernel = &gemm_sb_kernel<TYPE, BM, FFNP, SK, LO, LF>;
+  WH_ENSURE_LDS(lds, kernel);
   const dim3 grid(static_cast<unsigned>(SK ? a.sk_g : n_tiles), static_cast<unsigned>(SK ? 1 : a.splits));
   const int upw = SK ? (n_tiles * nsb + a.sk_g - 1) / a.sk_g : 0;
   const int sbps = (nsb + a.splits - 1) / a.splits;
-  gemm_sb_kernel<TYPE, BM, FFNP, SK, LO><<<grid, TWAVES * 64, lds, s>>>(
+  kernel<<<grid, TWAVES * 64, lds, s>>>(
       a.w, a.w2, a.frag, a.rs, a.bs, a.y, a.n_tokens, a.n_rows, nsb, sbps, tiles_n, n_tiles,
       a.sk_flags, a.sk_part, upw, a.sk_sub, a.sk_wait, sb_chain(BM, SK ? std::min(nsb, upw) : sbps));
   WH_LAUNCH_CHECK("k-quant gemm kernel launch");
@@ -587,6 +674,13 @@ int sb_launch_bm(const wh::SbGemm& a, hipStream_t s) {
       if (a.ffn) return sb_launch<TYPE, BM, true, true, true>(a, s);
       return a.lo ? sb_launch<TYPE, BM, false, true, true>(a, s) : sb_launch<TYPE, BM, false, true, false>(a, s);
     }
+  }
+  if constexpr (TYPE == wh::kGemmQ6S && BM <= 64) {
+    const int lf = sb_lo_first(TYPE, BM, a.n_tokens, (a.k / 256 + a.splits - 1) / a.splits, a.ffn);
+    if (lf && !a.lo) return sb_launch<TYPE, BM, false, false, false, 1>(a, s);
+    if (lf == 1) return sb_launch<TYPE, BM, false, false, true, 1>(a, s);
+    if constexpr (BM == 64)
+      if (lf == 2) return sb_launch<TYPE, BM, false, false, true, 2>(a, s);
   }
   if (a.ffn) return sb_launch<TYPE, BM, true, false, true>(a, s);
   return a.lo ? sb_launch<TYPE, BM, false, false, true>(a, s) : sb_launch<TYPE, BM, false, false, false>(a, s);

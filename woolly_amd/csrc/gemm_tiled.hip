@@ -835,21 +835,35 @@ __global__ __launch_bounds__(TWAVES * 64, 1) void gemm_tiled_kernel(
   }  // segment
 }
 
+// ACC double: the K-quants, whose up to 16 planes of a super-block or two each
+// would be rounded 15 times at the size of the sum (Q6_K 4096 x 4096 at 20
+// tokens: error 1.3e-7, 1.0e-7 with this and the order of sb_lo_first);
+// memory-bound either way.
+template <typename ACC>
 __global__ __launch_bounds__(256) void tiled_splitk_reduce_kernel(const float* __restrict__ part, int splits,
                                                                   size_t n, float* __restrict__ y) {
   const size_t stride = static_cast<size_t>(gridDim.x) * blockDim.x;
   for (size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += stride) {
-    float v = part[i];
+    ACC v = part[i];
     for (int s = 1; s < splits; s++) v += part[static_cast<size_t>(s) * n + i];
-    y[i] = v;
+    y[i] = static_cast<float>(v);
   }
 }
 
 // Token-tile height for a token count: the smallest of 16, 32, 64, 128 that
-// holds it (one tile) or 128 beyond.
-int tile_bm(int type, size_t n_tokens) {
+// holds it (one tile) or 128 beyond.  Q6_K stays at 64 where 128-token tiles
+// hold at most 1.5 super-blocks per CU: the sums are so short there that the
+// rounding of the products with lo limbs shows, which the 64-token kernel has
+// the registers to order (gemm_sb.hpp, sb_lo_first), and CUs would idle (2048 x
+// 1024 at 100 tokens: error 1.05e-7 and 27.0 us, with 64 0.86e-7 and 21.5 us;
+// 8192 x 3072 1.17e-7 and 43.3 us, 1.07e-7 and 38.8 us).
+int tile_bm(int type, size_t n_rows, size_t n_tokens, size_t k) {
   if (n_tokens <= 16 && !is_sb(type)) return 16;  // (the K-quant kernel starts at 32)
-  return n_tokens <= 32 ? 32 : (n_tokens <= 64 ? 64 : 128);
+  if (n_tokens <= 64) return n_tokens <= 32 ? 32 : 64;
+  if (type == wh::kGemmQ6S &&
+      (n_tokens + 127) / 128 * ((n_rows + TBN - 1) / TBN) * (k / 256) <= static_cast<size_t>(wh::cu_count()) * 3 / 2)
+    return 64;
+  return 128;
 }
 
 // Stream-K grid for n_tiles tiles of tile_st stages each: one workgroup per
@@ -970,7 +984,7 @@ int launch_ffn_bm(const uint8_t* gate, const uint8_t* up, size_t n_ff, size_t k,
 template <int TYPE>
 int launch_ffn_typed(const uint8_t* gate, const uint8_t* up, size_t n_ff, size_t k, size_t n_tokens,
                      const _Float16* frag, const float* rs, const float* bs, float* h, const SkWs& sk, hipStream_t s) {
-  switch (tile_bm(TYPE, n_tokens)) {
+  switch (tile_bm(TYPE, n_ff, n_tokens, k)) {
     case 16: return launch_ffn_bm<TYPE, 16>(gate, up, n_ff, k, n_tokens, frag, rs, bs, h, sk, s);
     case 32: return launch_ffn_bm<TYPE, 32>(gate, up, n_ff, k, n_tokens, frag, rs, bs, h, sk, s);
     case 64: return launch_ffn_bm<TYPE, 64>(gate, up, n_ff, k, n_tokens, frag, rs, bs, h, sk, s);
@@ -982,7 +996,7 @@ template <int TYPE>
 int launch_typed(const uint8_t* w, size_t n_rows, size_t k, size_t n_tokens, const _Float16* frag,
                  const float* rs, const float* bs, float* part, int splits, const SkWs& sk,
                  hipStream_t s, bool lo) {
-  switch (tile_bm(TYPE, n_tokens)) {
+  switch (tile_bm(TYPE, n_rows, n_tokens, k)) {
     case 16: return launch_bm<TYPE, 16>(w, n_rows, k, n_tokens, frag, rs, bs, part, splits, sk, s, lo);
     case 32: return launch_bm<TYPE, 32>(w, n_rows, k, n_tokens, frag, rs, bs, part, splits, sk, s, lo);
     case 64: return launch_bm<TYPE, 64>(w, n_rows, k, n_tokens, frag, rs, bs, part, splits, sk, s, lo);
@@ -1025,7 +1039,7 @@ static size_t tiled_ts(int type) {
 bool gemm_tiled_ok(int type, const void* w, const float* x, size_t n_rows, size_t k, size_t n_tokens) {
   const size_t ts = tiled_ts(type);
   if (ts == 0 || k == 0 || k % (32 * SB) != 0 || !aligned(w, 4) || !aligned(x, 16) || ((k / 32) * ts) % 4 != 0) return false;
-  const size_t bm = static_cast<size_t>(tile_bm(type, n_tokens));
+  const size_t bm = static_cast<size_t>(tile_bm(type, n_rows, n_tokens, k));
   const size_t tm = (n_tokens + bm - 1) / bm * bm;
   const size_t lim = static_cast<size_t>(1) << 32;
   if (n_rows * (k / 32) * ts >= lim || tm * k * 4 >= lim) return false;
@@ -1045,7 +1059,7 @@ bool gemm_tiled_ok(int type, const void* w, const float* x, size_t n_rows, size_
 // kernel: 16, and one super-block; planes that whole super-blocks per split
 // would leave empty are not formed: 17 super-blocks in 16 splits are 9 of two).
 int gemm_tiled_splits(int type, size_t n_rows, size_t n_tokens, size_t k) {
-  const size_t bm = static_cast<size_t>(tile_bm(type, n_tokens));
+  const size_t bm = static_cast<size_t>(tile_bm(type, n_rows, n_tokens, k));
   const size_t tiles = ((n_rows + TBN - 1) / TBN) * ((n_tokens + bm - 1) / bm);
   const size_t nb = k / 32;
   const size_t cus = static_cast<size_t>(cu_count());
@@ -1067,9 +1081,12 @@ int gemm_tiled_splits(int type, size_t n_rows, size_t n_tokens, size_t k) {
 // hand-off of a partial tile costs more than the reduce it replaces (M=32,
 // 14336 x 4096: 31.9 against 31.3 us).
 static int sk_plain(int type, size_t n_rows, size_t n_tokens, size_t k) {
-  const size_t bm = static_cast<size_t>(tile_bm(type, n_tokens));
+  const size_t bm = static_cast<size_t>(tile_bm(type, n_rows, n_tokens, k));
   const size_t tiles = ((n_tokens + bm - 1) / bm) * ((n_rows + TBN - 1) / TBN);
-  if (is_sb(type)) return sb_sk_grid(tiles, k / 256, static_cast<int>(bm), gemm_tiled_splits(type, n_rows, n_tokens, k));
+  if (is_sb(type)) {
+    if (bm == 64 && n_tokens > 64) return 0;  // short sums (tile_bm): split-K
+    return sb_sk_grid(tiles, k / 256, static_cast<int>(bm), gemm_tiled_splits(type, n_rows, n_tokens, k));
+  }
   return bm < 64 ? 0 : sk_grid(tiles, k / 32 / SB);
 }
 // Split-K factor of the GEMM over n_rows rows: 1 where it runs stream-K.
@@ -1079,28 +1096,28 @@ static int tiled_splits(int type, size_t n_rows, size_t n_tokens, size_t k) {
 static int sk_slots(int type, size_t n_rows, size_t n_tokens, size_t k) {
   const int g = sk_plain(type, n_rows, n_tokens, k);
   if (g) return g;
-  if (gemm_tiled_splits(type, 2 * n_rows, n_tokens, k) == 1 && tile_bm(type, n_tokens) >= 64) {
-    const size_t bm = static_cast<size_t>(tile_bm(type, n_tokens));
+  if (gemm_tiled_splits(type, 2 * n_rows, n_tokens, k) == 1 && tile_bm(type, n_rows, n_tokens, k) >= 64) {
+    const size_t bm = static_cast<size_t>(tile_bm(type, n_rows, n_tokens, k));
     const size_t tiles = ((n_tokens + bm - 1) / bm) * ((n_rows + TBN / 2 - 1) / (TBN / 2));
     return is_sb(type) ? sb_sk_grid(tiles, k / 256, static_cast<int>(bm), 1) : sk_grid(tiles, k / 32 / SB);
   }
   return 0;
 }
 
-static size_t sk_bytes(int type, int slots, size_t n_tokens) {
+static size_t sk_bytes(int slots, size_t bm) {
   return slots ? al256(static_cast<size_t>(slots) * 4) +
-                     static_cast<size_t>(slots) * static_cast<size_t>(tile_bm(type, n_tokens)) * TBN * 4
+                     static_cast<size_t>(slots) * bm * TBN * 4
                : 0;
 }
 
 size_t gemm_tiled_workspace_bytes(int type, size_t n_rows, size_t n_tokens, size_t k) {
-  const size_t bm = static_cast<size_t>(tile_bm(type, n_tokens));
+  const size_t bm = static_cast<size_t>(tile_bm(type, n_rows, n_tokens, k));
   const size_t tm = (n_tokens + bm - 1) / bm * bm;   // padded tokens
   size_t b = al256(tm * k * 4) + al256(tm * 4);
   if (needs_bsum(type)) b += al256(tm * bsum_groups(type, k) * 4);
   const int splits = tiled_splits(type, n_rows, n_tokens, k);
   if (splits > 1) b += al256(static_cast<size_t>(splits) * n_rows * n_tokens * 4);
-  return b + sk_bytes(type, sk_slots(type, n_rows, n_tokens, k), n_tokens);
+  return b + sk_bytes(sk_slots(type, n_rows, n_tokens, k), bm);
 }
 
 // Workspace of one tiled GEMM: packed activations, row scales, Q4_1 block
@@ -1119,7 +1136,7 @@ struct TiledWs {
 
 static TiledWs tiled_ws(int type, size_t n_rows, size_t k, size_t n_tokens, void* workspace) {
   TiledWs t{};
-  t.bm = tile_bm(type, n_tokens);
+  t.bm = tile_bm(type, n_rows, n_tokens, k);
   t.tm = (n_tokens + t.bm - 1) / t.bm * t.bm;
   char* ws = static_cast<char*>(workspace);
   t.frag = reinterpret_cast<_Float16*>(ws);
@@ -1209,7 +1226,8 @@ static int tiled_run(int type, const void* w, size_t n_rows, size_t k, size_t n_
     size_t gsz = (n + 255) / 256;
     const size_t cap = static_cast<size_t>(cu_count()) * 8;
     if (gsz > cap) gsz = cap;
-    tiled_splitk_reduce_kernel<<<static_cast<unsigned>(gsz), 256, 0, s>>>(part, t.splits, n, y);
+    auto* reduce = is_sb(type) ? tiled_splitk_reduce_kernel<double> : tiled_splitk_reduce_kernel<float>;
+    reduce<<<static_cast<unsigned>(gsz), 256, 0, s>>>(part, t.splits, n, y);
     WH_LAUNCH_CHECK("split-K reduce launch");
   }
   return WH_OK;
