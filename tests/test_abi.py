@@ -229,21 +229,24 @@ def test_kquant_split_k_has_no_empty_planes(t, nsb, planes):
         up(conv) + up(tm * k * 4) + up(tm * 4) + sums + up(planes * n * m * 4)
 
 
-@pytest.mark.parametrize("t", [12, 14])
-@pytest.mark.parametrize("n,k,m,planes", [
-    (1280, 14336, 100, 14), (3072, 5632, 90, 11), (4096, 4352, 70, 9), (512, 14336, 300, 14),  # many owners: split-K
-    (14336, 8192, 100, 4),                                    # seven super-blocks of eight: split-K
-    (10240, 5632, 100, 0), (20480, 4096, 100, 0),             # four of six, five of eight: stream-K
-    (16384, 2048, 60, 0), (14336, 4096, 512, 0)])             # 64-token tiles; without split-K
-def test_kquant_stream_k_or_split_k(t, n, k, m, planes):
+@pytest.mark.parametrize("n,k,m,q4k,q6k", [  # planes of either type
+    (1280, 14336, 100, 14, 14), (3072, 5632, 90, 11, 8), (4096, 4352, 70, 9, 6), (512, 14336, 300, 14, 14),  # many owners
+    (14336, 8192, 100, 4, 4),                                 # seven super-blocks of eight: split-K
+    (10240, 5632, 100, 0, 0), (20480, 4096, 100, 0, 0),       # four of six, five of eight: stream-K
+    (16384, 2048, 60, 0, 0), (14336, 4096, 512, 0, 0)])       # 64-token tiles; without split-K
+def test_kquant_stream_k_or_split_k(n, k, m, q4k, q6k):
     """The workspace shows which the plan takes: split-K planes, or (0 here) a
     slot of one tile and a flag for each of the 256 CUs that a machine without
-    a GPU plans for."""
+    a GPU plans for.  Q6_K takes 64-token tiles where 128-token ones hold up to
+    1.5 super-blocks per CU (the first four)."""
     lib = _lib.load()
     up = lambda v: (v + 255) // 256 * 256
-    nsb, bm = k // 256, 64 if m <= 64 else 128
-    tm = -(-m // bm) * bm
-    conv = n * (k // 64 * 40 + (nsb + 7) // 8 * 16 if t == 12 else k // 64 * 80)
-    sums = up(tm * ((nsb + 7) // 8 * 8) * 4) if t == 12 else 0
-    got = lib.wh_quantized_matmul_workspace_bytes(t, n, k, m) - (up(conv) + up(tm * k * 4) + up(tm * 4) + sums)
-    assert got == (up(planes * n * m * 4) if planes else 256 * 4 + 256 * bm * 256 * 4)
+    nsb = k // 256
+    for t, planes in ((12, q4k), (14, q6k)):
+        short = t == 14 and -(-m // 128) * -(-n // 256) * nsb <= 384
+        bm = 64 if m <= 64 or short else 128
+        tm = -(-m // bm) * bm
+        conv = n * (k // 64 * 40 + (nsb + 7) // 8 * 16 if t == 12 else k // 64 * 80)
+        sums = up(tm * ((nsb + 7) // 8 * 8) * 4) if t == 12 else 0
+        got = lib.wh_quantized_matmul_workspace_bytes(t, n, k, m) - (up(conv) + up(tm * k * 4) + up(tm * 4) + sums)
+        assert got == (up(planes * n * m * 4) if planes else 256 * 4 + 256 * bm * 256 * 4), t
