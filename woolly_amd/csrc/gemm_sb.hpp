@@ -11,8 +11,12 @@
 // that FMA comes once per step and the scale's product with it, which made the
 // vector ALU the bound (3.4 VALU operations per MFMA), and Q6_K's
 // 16-element groups had to be padded with zeros to 32 (four products per
-// 32 elements; here three: x_lo w_hi, x_hi w_hi, x_hi w_lo; the x_lo w_lo
-// left out is below 2^-23 of x w, and x itself carries 22 bits).
+// 32 elements; here three: x_lo w_hi, x_hi w_lo, x_hi w_hi; the x_lo w_lo left
+// out is at most 2^-22 of x w, where |s (q - 32)| > 2048, and x itself carries 22
+// bits.  Products that all have one sign show it: 2.4e-7 in sums of four
+// super-blocks and 3.4e-7 in sums of four with K = 14336, where the 16-element
+// blocks had 3.8e-7 and 1.4e-6 from their longer f32 sums.  In shorter sums it
+// is formed: sb_lo_first).
 // Activations are fp16 hi + lo of the row scaled by a power of two, as in
 // gemm_tiled.hip (its pack_a_kernel writes them).
 //
@@ -66,22 +70,18 @@ constexpr int sb_rec() { return TYPE == wh::kGemmQ4S ? 40 : 80; }  // bytes per 
 // us with 64, 120.6 with 128; at M=128 55.1 and 53.5.
 inline int sb_chain(int bm, int sb) { return bm == 128 && sb >= 8 ? 1 : 0; }
 
-// Q6_K where a workgroup sums one or two super-blocks: the products with an x_lo
-// or w_lo of both steps of a stage come before the x_hi w_hi of either (1).  An
-// MFMA rounds four times at the size of C, and the two products of lo limbs
-// between the x_hi w_hi of the two steps are most of a short sum's error.
-// 2: x_lo w_lo too, in the 64-token tiles of a longer prompt (gemm_tiled.hip's
-// tile_bm: up to four super-blocks).  Error against 64
-// bits (with 0; with one scale per 16 elements, whose quants are exact), 1e-7:
-// 2048 x 1024 at 20 and 64 tokens 0.93 (1.07; 0.98), at 100 0.86 (1.08; 1.00),
-// 1024 x 2048 at 50 0.97 (1.18; 1.08), 4096 x 4096 at 20 1.02 (1.34; 1.32).  Time
-// 2048 x 1024 at 20 tokens 14.0 us (13.7), 14336 x 1024 at 64 26.6 us (26.1); the
-// longer sums of 14336 x 4096 do not need it (1.29; 1.59) and would take 29.3 us
-// instead of 28.2 at 32 tokens.
-inline int sb_lo_first(int type, int bm, int n_tokens, int sb, bool ffn) {
-  if (type != wh::kGemmQ6S || bm > 64 || ffn) return 0;
-  if (n_tokens > 64) return 2;
-  return sb <= 2 ? 1 : 0;
+// Q6_K where a workgroup sums one or two super-blocks, and the 64-token tiles of
+// longer prompts (gemm_tiled.hip's tile_bm; up to four): the products with an
+// x_lo or w_lo of both steps of a stage, x_lo w_lo among them, come before the
+// x_hi w_hi of either.  An MFMA rounds four times at the size of C, and the two
+// products of lo limbs between the x_hi w_hi of the two steps are most of a short
+// sum's error.  Against 64 bits (without; with one scale per 16 elements, whose
+// quants are exact), 1e-7: 2048 x 1024 at 20 and 64 tokens 0.85 (1.07; 0.98), 1024 x
+// 2048 at 50 0.89 (1.18; 1.08), 4096 x 4096 at 20 0.94 (1.34; 1.32).  Time 2048 x 1024
+// at 20 tokens 14.4 us (13.9), 14336 x 1024 at 64 27.3 us (25.8); the longer sums of
+// 14336 x 4096 do not need it (1.29; 1.59) and would take 30.6 us instead of 28.2.
+inline bool sb_lo_first(int type, int bm, int n_tokens, int sb, bool ffn) {
+  return type == wh::kGemmQ6S && bm <= 64 && !ffn && (n_tokens > 64 || sb <= 2);
 }
 
 template <int TYPE, int BM, bool LO>
@@ -110,7 +110,7 @@ __device__ __forceinline__ half2v sb_nib(uint32_t u, uint32_t mask, half2v s) {
 
 // Weight rows r0.. of one tile, K stages [st_a, st_b): the GEMM over it.  Grid
 // and stream-K (SK) as gemm_tiled_kernel; units are super-blocks.
-template <int TYPE, int BM, bool FFNP, bool SK, bool LO, int LF>
+template <int TYPE, int BM, bool FFNP, bool SK, bool LO, bool LF>
 __global__ __launch_bounds__(TWAVES * 64, 1) void gemm_sb_kernel(
     const uint8_t* __restrict__ W, const uint8_t* __restrict__ W2, const _Float16* __restrict__ frag,
     const float* __restrict__ rscale, const float* __restrict__ bsum, float* __restrict__ y, int n_tokens, int n_rows,
@@ -352,7 +352,7 @@ __global__ __launch_bounds__(TWAVES * 64, 1) void gemm_sb_kernel(
         asm volatile("" ::: "memory");
         issue();
       };
-      if constexpr (LF != 0) {
+      if constexpr (LF) {
         auto step = [&](half8 (&a)[IT], half8 (&b)[NT], auto then) {
 #pragma unroll
           for (int n = 0; n < NT; n++) {
@@ -377,10 +377,10 @@ __global__ __launch_bounds__(TWAVES * 64, 1) void gemm_sb_kernel(
           form_lo(n);
           __builtin_amdgcn_sched_barrier(0);
         }
-        // its x_hi w_lo; the second step's weights formed and its x_hi read
+        // its x_lo w_lo and x_hi w_lo; the second step's weights formed and its x_hi read
         read_a(slot, 1, 0, ah1);
         if (tail) read_d(slot);
-        if constexpr (LO && LF == 2) step(al, bl, [](int) {});
+        if constexpr (LO) step(al, bl, [](int) {});
         step(ah, bl, [&](int n) {
           rq[n] = rq1[n];
 #pragma unroll
@@ -408,7 +408,7 @@ __global__ __launch_bounds__(TWAVES * 64, 1) void gemm_sb_kernel(
         turn();
         read_q(nslot, 0);
         read_s(nslot);
-        if constexpr (LO && LF == 2) step(al1, bl, [](int) {});
+        if constexpr (LO) step(al1, bl, [](int) {});
         step(ah1, bl, [](int) {});
         // x_hi w_hi of both; the next stage's x_lo read and weights formed
         if constexpr (LO) read_a(nslot, 0, 1, al);
@@ -649,7 +649,7 @@ __global__ __launch_bounds__(TWAVES * 64, 1) void gemm_sb_kernel(
   }  // segment
 }
 
-template <int TYPE, int BM, bool FFNP, bool SK, bool LO, int LF = 0>
+template <int TYPE, int BM, bool FFNP, bool SK, bool LO, bool LF = false>
 int sb_launch(const wh::SbGemm& a, hipStream_t s) {
   const int tiles_n = (a.n_rows + (FFNP ? TBN / 2 : TBN) - 1) / (FFNP ? TBN / 2 : TBN);
   const int n_tiles = (a.n_tokens + BM - 1) / BM * tiles_n;
@@ -676,11 +676,8 @@ int sb_launch_bm(const wh::SbGemm& a, hipStream_t s) {
     }
   }
   if constexpr (TYPE == wh::kGemmQ6S && BM <= 64) {
-    const int lf = sb_lo_first(TYPE, BM, a.n_tokens, (a.k / 256 + a.splits - 1) / a.splits, a.ffn);
-    if (lf && !a.lo) return sb_launch<TYPE, BM, false, false, false, 1>(a, s);
-    if (lf == 1) return sb_launch<TYPE, BM, false, false, true, 1>(a, s);
-    if constexpr (BM == 64)
-      if (lf == 2) return sb_launch<TYPE, BM, false, false, true, 2>(a, s);
+    if (sb_lo_first(TYPE, BM, a.n_tokens, (a.k / 256 + a.splits - 1) / a.splits, a.ffn))
+      return a.lo ? sb_launch<TYPE, BM, false, false, true, true>(a, s) : sb_launch<TYPE, BM, false, false, false, true>(a, s);
   }
   if (a.ffn) return sb_launch<TYPE, BM, true, false, true>(a, s);
   return a.lo ? sb_launch<TYPE, BM, false, false, true>(a, s) : sb_launch<TYPE, BM, false, false, false>(a, s);
