@@ -233,6 +233,7 @@ def test_kquant_split_k_has_no_empty_planes(t, nsb, planes):
     (1280, 14336, 100, 14, 14), (3072, 5632, 90, 11, 8), (4096, 4352, 70, 9, 6), (512, 14336, 300, 14, 14),  # many owners
     (14336, 8192, 100, 4, 4),                                 # seven super-blocks of eight: split-K
     (10240, 5632, 100, 0, 0), (20480, 4096, 100, 0, 0),       # four of six, five of eight: stream-K
+    (28672, 4096, 100, 0, 0),                                 # two splits: seven of eight too
     (16384, 2048, 60, 0, 0), (14336, 4096, 512, 0, 0)])       # 64-token tiles; without split-K
 def test_kquant_stream_k_or_split_k(n, k, m, q4k, q6k):
     """The workspace shows which the plan takes: split-K planes, or (0 here) a

@@ -888,14 +888,15 @@ int sk_grid(size_t n_tiles, size_t tile_st) {
 // of six: 56.1 / 62.9; 80 of 16, five of eight: 64.8 / 73.3), and not below that
 // (56 of 32, seven of eight: 84.2 / 77.4; 64 of 22, six of six: 73.9 / 69.5).
 // 64-token tiles hand over half as much: they gain with up to four in any case
-// (60 tokens, 64 of 8: 27.0 / 28.8; 64 of 22 47.1 / 45.6).  Without split-K it
-// needs any shortening.
+// (60 tokens, 64 of 8: 27.0 / 28.8; 64 of 22 47.1 / 45.6).  Against one or two
+// splits it needs any shortening (100 tiles of 13, six of seven: 68.9 / 72.2; 112
+// of 16, seven of eight: 73.4 / 74.0).
 int sb_sk_grid(size_t n_tiles, size_t nsb, int bm, int splits) {
   const size_t g = static_cast<size_t>(wh::cu_count());
   if (g == 0 || g % 8 != 0 || n_tiles % g == 0 || bm < 64 || splits > 4) return 0;
   const size_t upw = (n_tiles * nsb + g - 1) / g;
   const size_t per = (n_tiles * splits + g - 1) / g * ((nsb + splits - 1) / splits);
-  const bool gain = splits == 1 ? upw < per : bm == 64 || 8 * upw < 7 * per;
+  const bool gain = splits <= 2 ? upw < per : bm == 64 || 8 * upw < 7 * per;
   return upw >= 2 && gain ? static_cast<int>(g) : 0;
 }
 
