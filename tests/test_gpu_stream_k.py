@@ -25,6 +25,7 @@ from woolly_amd.device import DeviceBuffer
 pytestmark = pytest.mark.gpu
 Q4_0, Q4_1, Q8_0, Q4_K, Q6_K = 2, 3, 8, 12, 14
 REL_L2 = 1e-4
+KQ_REL_L2 = 2e-6  # k roundings of f32 sums of the terms' size; a lost lo limb costs 1e-4
 
 
 def max_abs_bar(ref) -> float:
@@ -90,9 +91,10 @@ def test_stream_k_matmul(gpu, orc, t, n, k, m):
 @pytest.mark.parametrize("t", [Q4_K, Q6_K])
 @pytest.mark.parametrize("n,k,m", [(14336, 4096, 512), (4096, 14336, 100)])
 def test_stream_k_kquant_matmul(gpu, orc, t, n, k, m):
-    """The K-quant formats (converted per call to 32-element blocks with f32
-    scales): the same split, Q4_K's dmin term added once per tile by the
-    workgroup that finishes it."""
+    """The K-quant formats (converted per call to stage records): two owners
+    per shared tile at M=512, Q4_K's dmin term added once per tile by the
+    workgroup that finishes it; the second shape, whose tiles would have 14
+    owners, takes split-K."""
     print(f"[case] stream-K kquant matmul type={t} m={m} n={n} k={k}", flush=True)
     w = synth.quantized_weight(t, n, k, seed=n + k + t)
     x = synth.activations(m * k, seed=m + t).reshape(m, k)
@@ -104,7 +106,67 @@ def test_stream_k_kquant_matmul(gpu, orc, t, n, k, m):
     got = outs[0][rows]
     r, a = rel_l2(got, ref), max_abs(got, ref)
     report(f"stream-K kquant matmul t={t} m={m} n={n} k={k}", r, a, ref)
-    assert r <= REL_L2 and a <= max_abs_bar(ref)
+    assert r <= KQ_REL_L2 and a <= max_abs_bar(ref)
+
+
+# (n, k, m), super-blocks per workgroup of a tile's: 80 tiles 5 of 16, 40 tiles 4 of
+# 22, 64 tiles of 64 tokens 2 of 8 and 8 of 32, 168 tiles 11 of 16
+KQ_PARTS = [(20480, 4096, 100), (10240, 5632, 100), (16384, 2048, 60), (16384, 8192, 60), (14336, 4096, 300)]
+
+
+@pytest.mark.parametrize("t", [Q4_K, Q6_K])
+@pytest.mark.parametrize("n,k,m", KQ_PARTS)
+@pytest.mark.parametrize("wait", [None, 0])
+def test_stream_k_kquant_parts(gpu, orc, t, n, k, m, wait):
+    """K-quant tiles of 64 and 128 tokens with up to six owners, handed over or
+    (wait bound 0) computed by the finishing workgroup in a second pass.  Q4_K:
+    dmin of -128 to -512 d, against activations with a mean of 0.5, carries most of
+    each output, so a part's end inside the 32-super-block windows shows."""
+    print(f"[case] stream-K kquant parts type={t} m={m} n={n} k={k} wait={wait}", flush=True)
+    w = synth.quantized_weight(t, n, k, seed=n + k + t)
+    if t == Q4_K:
+        b = w.reshape(-1, 144)
+        d = b[:, 12:14].copy().view(np.float16).astype(np.float32)[:, 0]
+        mult = np.random.default_rng(n).uniform(-512.0, -128.0, size=d.shape)
+        b[:, 14:16] = (np.abs(d) * mult).astype(np.float16).view(np.uint8).reshape(-1, 2)
+    x = synth.activations(m * k, seed=m + t, mean=0.5).reshape(m, k)
+    try:
+        if wait is not None:
+            ops.set_stream_k_wait(wait)
+        outs = run_matmul(t, w, n, k, x, m)
+    finally:
+        ops.set_stream_k_wait(ops.STREAM_K_WAIT_DEFAULT)
+    rows = np.array([r for r in ROWS if r < m], dtype=np.int64)
+    ref = orc.matmul_rows_f64(t, w, n, k, x, m, rows)
+    for o in outs:
+        assert wait == 0 or np.array_equal(o, outs[0]), "repeated calls differ"
+        assert rel_l2(o[rows], ref) <= KQ_REL_L2
+    report(f"stream-K kquant parts t={t} m={m} n={n} k={k} wait={wait}", rel_l2(outs[0][rows], ref),
+           max_abs(outs[0][rows], ref), ref)
+
+
+@pytest.mark.parametrize("t", [Q4_K, Q6_K])
+@pytest.mark.parametrize("hidden,n_ff,m", [(4096, 14336, 200), (1024, 20480, 60)])
+@pytest.mark.parametrize("wait", [None, 0])
+def test_stream_k_kquant_ffn(gpu, orc, t, hidden, n_ff, m, wait):
+    """Gate and up in one pass under stream-K, in tiles of 128 and of 64 tokens."""
+    print(f"[case] stream-K kquant ffn type={t} hidden={hidden} n_ff={n_ff} m={m} wait={wait}", flush=True)
+    L = synth.ffn_layer(t, hidden, n_ff, m, seed=hidden + n_ff + t)
+    bufs = {key: up(v) for key, v in L.items()}
+    ob = DeviceBuffer(4 * m * hidden)
+    wsz = ops.ffn_workspace_bytes(hidden, n_ff, m, ggml_type=t)
+    ws = DeviceBuffer(wsz)
+    try:
+        if wait is not None:
+            ops.set_stream_k_wait(wait)
+        ops.ffn_swiglu(t, bufs["gate"][1], bufs["up"][1], bufs["down"][1], hidden, n_ff,
+                       bufs["gamma"][1], 1e-5, bufs["x"][1], m, ob.ptr, ws.ptr, wsz)
+        got = down(ob, np.float32, m * hidden).reshape(m, hidden)
+    finally:
+        ops.set_stream_k_wait(ops.STREAM_K_WAIT_DEFAULT)
+    rows = [r for r in (0, 1, 59, 127, 128, 199) if r < m]
+    ref = orc.ffn_rows_f64(t, L["gate"], L["up"], L["down"], hidden, n_ff, L["gamma"], 1e-5, L["x"], rows)
+    assert rel_l2(got[rows], ref) <= 2 * KQ_REL_L2   # two products behind each other
 
 
 def test_stream_k_shapes_cover_three_owners():

@@ -80,8 +80,14 @@ inline int sb_chain(int bm, int sb) { return bm == 128 && sb >= 8 ? 1 : 0; }
 // 2048 at 50 0.89 (1.18; 1.08), 4096 x 4096 at 20 0.94 (1.34; 1.32).  Time 2048 x 1024
 // at 20 tokens 14.4 us (13.9), 14336 x 1024 at 64 27.3 us (25.8); the longer sums of
 // 14336 x 4096 do not need it (1.29; 1.59) and would take 30.6 us instead of 28.2.
+// Q4_K, whose products are exact fp16s, has two products per step; it takes this
+// order in the FFN's gate and up of up to seven super-blocks in 128-token tiles,
+// where one pass sums twice as far as two passes in split-K did (FFN 1536 x 4096
+// at 804 tokens 4.87e-7 -> 4.78e-7, in the same time; its stream-K kernel has no
+// registers left for it).
 inline bool sb_lo_first(int type, int bm, int n_tokens, int sb, bool ffn) {
-  return type == wh::kGemmQ6S && bm <= 64 && !ffn && (n_tokens > 64 || sb <= 2);
+  if (type == wh::kGemmQ4S) return ffn && bm == 128 && sb < 8;
+  return bm <= 64 && !ffn && (n_tokens > 64 || sb <= 2);
 }
 
 template <int TYPE, int BM, bool LO>
@@ -116,7 +122,7 @@ __global__ __launch_bounds__(TWAVES * 64, 1) void gemm_sb_kernel(
     const float* __restrict__ rscale, const float* __restrict__ bsum, float* __restrict__ y, int n_tokens, int n_rows,
     int nsb, int sb_per_split, int tiles_n, int n_tiles, uint32_t* __restrict__ sk_flags, float* __restrict__ sk_part,
     int sk_upw, int sk_sub, uint32_t sk_wait,
-    int chain) {
+    int chain, bool parts) {
   using C = SbCfg<BM>;
   using S = SbStage<TYPE, BM, LO>;
   constexpr int IT = C::IT, NT = C::NT, REC = sb_rec<TYPE>(), N = S::N;
@@ -352,7 +358,54 @@ __global__ __launch_bounds__(TWAVES * 64, 1) void gemm_sb_kernel(
         asm volatile("" ::: "memory");
         issue();
       };
-      if constexpr (LF) {
+      if constexpr (LF && Q4) {
+        // x_lo of both steps, then x_hi of both: one operand set read while the
+        // other is multiplied, the second step's weights in bw1
+        auto form1 = [&](int n) {
+          const uint32_t q = rq[n].y;
+          const half2v s16 = sc[n] * half2v{static_cast<_Float16>(0.0625f), static_cast<_Float16>(0.0625f)};
+          const half2v p[4] = {sb_nib(q, 0x000F000Fu, sc[n]), sb_nib(q, 0x00F000F0u, s16),
+                               sb_nib(q >> 8, 0x000F000Fu, sc[n]), sb_nib(q >> 8, 0x00F000F0u, s16)};
+#pragma unroll
+          for (int c = 0; c < 4; c++) {
+            bw1[n][2 * c] = p[c][0];
+            bw1[n][2 * c + 1] = p[c][1];
+          }
+        };
+        auto phase = [&](half8 (&a)[IT], half8 (&b)[NT], auto then) {
+#pragma unroll
+          for (int n = 0; n < NT; n++) {
+#pragma unroll
+            for (int i = 0; i < IT; i++) mma(i, n, a[i], b[n]);
+            then(n);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+        };
+        read_a(slot, 1, 1, ah);
+        phase(al, bw, [&](int n) {
+          if (head && n == 0) apply(NT - 1, dn[NT - 1]);
+          if (n < NT / 2) form(n + NT / 2, 0);
+          else form1(n - NT / 2);
+        });
+        read_a(slot, 0, 0, al);
+        phase(ah, bw1, [&](int n) {
+          if (n < NT / 2) form1(n + NT / 2);
+        });
+        read_a(slot, 1, 0, ah);
+        if (tail) read_d(slot);
+        phase(al, bw, [](int) {});
+        turn();
+        read_q(nslot, 0);
+        read_s(nslot);
+        read_a(nslot, 0, 1, al);
+        phase(ah, bw1, [&](int n) {
+          if (tail && n > 0) apply(n - 1, dn[n - 1]);
+          if (n >= NT / 2) form(n - NT / 2, 0);
+        });
+        cur = nxt;
+        continue;
+      }
+      if constexpr (LF && !Q4) {
         auto step = [&](half8 (&a)[IT], half8 (&b)[NT], auto then) {
 #pragma unroll
           for (int n = 0; n < NT; n++) {
@@ -495,6 +548,65 @@ __global__ __launch_bounds__(TWAVES * 64, 1) void gemm_sb_kernel(
       cur = nxt;
   }
   apply(NT - 1, dn[NT - 1]);
+  if constexpr (Q4) {
+    // dmin: acc += dmin[row][sb] S[token][sb] over the super-blocks just summed
+    // (stream-K: see sb_launch), as matrix-core products over windows of 32 super-blocks: lane group g
+    // holds super-blocks 8g .. 8g + 7 of the window in both operands (B: the
+    // fp16 table behind the records, those of other splits masked to zero; A:
+    // the packing's sums as hi + lo fp16 limbs of S 2^-10).
+    const int nsbp = (nsb + 7) & ~7;
+    const bool own = !SK || parts;
+    const int sb_lo = own ? sb0 : 0, sb_hi = own ? (pass ? nsb : sb_b) : (pass == 0 && sb_a == 0 ? nsb : 0);
+    const size_t table = static_cast<size_t>(nsb) * 4 * stage_stride;
+    const uint16_t* dm1 = reinterpret_cast<const uint16_t*>(W + table);
+    const uint16_t* dm2 = FFNP ? reinterpret_cast<const uint16_t*>(W2 + table) : dm1;
+    const uint16_t* s16 = reinterpret_cast<const uint16_t*>(bsum);
+    // opaque, so that the loads' offsets are formed here and not held in
+    // registers through the stage loop
+    int lnv = ln;
+    asm volatile("" : "+v"(lnv));
+    for (int w0 = sb_lo & ~31; w0 < sb_hi; w0 += 32) {
+      const int s0 = w0 + 8 * g;
+      const bool in = s0 < nsbp;
+      uint32_t mk[4];
+#pragma unroll
+      for (int d = 0; d < 4; d++) {
+        const int a = s0 + 2 * d;
+        mk[d] = (a >= sb_lo && a < sb_hi ? 0x0000FFFFu : 0u) | (a + 1 >= sb_lo && a + 1 < sb_hi ? 0xFFFF0000u : 0u);
+      }
+      u32x4 bd[NT];
+#pragma unroll
+      for (int n = 0; n < NT; n++) {
+        const int row = r0 + (FFNP ? wn / 2 + 16 * (n >> 1) : wn + 16 * n) + lnv;
+        const uint32_t off = static_cast<uint32_t>(min(row, n_rows - 1) * nsbp + s0);
+        bd[n] = in ? *reinterpret_cast<const u32x4*>(((n & 1) ? dm2 : dm1) + off) : u32x4{0u, 0u, 0u, 0u};
+      }
+      u32x4 sh[IT], sl[IT];
+#pragma unroll
+      for (int i = 0; i < IT; i++) {
+        const uint32_t off = static_cast<uint32_t>((t0 + wm + 16 * i + lnv) * 2 * nsbp + s0);
+        sh[i] = in ? *reinterpret_cast<const u32x4*>(s16 + off) : u32x4{0u, 0u, 0u, 0u};
+        sl[i] = in ? *reinterpret_cast<const u32x4*>(s16 + off + nsbp) : u32x4{0u, 0u, 0u, 0u};
+      }
+      __builtin_amdgcn_sched_barrier(0);  // every load issued before the first use
+#pragma unroll
+      for (int n = 0; n < NT; n++)
+#pragma unroll
+        for (int d = 0; d < 4; d++) bd[n][d] &= mk[d];
+#pragma unroll
+      for (int i = 0; i < IT; i++) {
+#pragma unroll
+        for (int n = 0; n < NT; n++) {
+          float4v t = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, sh[i]), __builtin_bit_cast(half8, bd[n]),
+                                                             float4v{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+          t = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, sl[i]), __builtin_bit_cast(half8, bd[n]), t, 0, 0, 0);
+#pragma unroll
+          for (int r = 0; r < 4; r++) acc[i][n][r] = __builtin_fmaf(1024.f, t[r], acc[i][n][r]);
+        }
+        __builtin_amdgcn_sched_barrier(0);  // one token group's products at a time
+      }
+    }
+  }
   if constexpr (!SK) break;
   if (pass > 0 || sb_a > 0 || sb_b == nsb) break;  // a tail part, the whole tile, or done here
   // head part: wait for the owners of the rest of the tile, then add their slots in order
@@ -544,66 +656,6 @@ __global__ __launch_bounds__(TWAVES * 64, 1) void gemm_sb_kernel(
       if (threadIdx.x == 0)
         __hip_atomic_store(sk_flags + v, static_cast<uint32_t>(sk_sub + 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       continue;
-    }
-  }
-
-  if constexpr (Q4) {
-    // dmin: acc += dmin[row][sb] S[token][sb] over the super-blocks of this
-    // split (stream-K: all of them, by the workgroup that finishes the tile),
-    // as matrix-core products over windows of 32 super-blocks: lane group g
-    // holds super-blocks 8g .. 8g + 7 of the window in both operands (B: the
-    // fp16 table behind the records, those of other splits masked to zero; A:
-    // the packing's sums as hi + lo fp16 limbs of S 2^-10).
-    const int nsbp = (nsb + 7) & ~7;
-    const int sb_lo = SK ? 0 : sb_a, sb_hi = SK ? nsb : sb_b;
-    const size_t table = static_cast<size_t>(nsb) * 4 * stage_stride;
-    const uint16_t* dm1 = reinterpret_cast<const uint16_t*>(W + table);
-    const uint16_t* dm2 = FFNP ? reinterpret_cast<const uint16_t*>(W2 + table) : dm1;
-    const uint16_t* s16 = reinterpret_cast<const uint16_t*>(bsum);
-    // opaque, so that the loads' offsets are formed here and not held in
-    // registers through the stage loop
-    int lnv = ln;
-    asm volatile("" : "+v"(lnv));
-    for (int w0 = sb_lo & ~31; w0 < sb_hi; w0 += 32) {
-      const int s0 = w0 + 8 * g;
-      const bool in = s0 < nsbp;
-      uint32_t mk[4];
-#pragma unroll
-      for (int d = 0; d < 4; d++) {
-        const int a = s0 + 2 * d;
-        mk[d] = (a >= sb_lo && a < sb_hi ? 0x0000FFFFu : 0u) | (a + 1 >= sb_lo && a + 1 < sb_hi ? 0xFFFF0000u : 0u);
-      }
-      u32x4 bd[NT];
-#pragma unroll
-      for (int n = 0; n < NT; n++) {
-        const int row = r0 + (FFNP ? wn / 2 + 16 * (n >> 1) : wn + 16 * n) + lnv;
-        const uint32_t off = static_cast<uint32_t>(min(row, n_rows - 1) * nsbp + s0);
-        bd[n] = in ? *reinterpret_cast<const u32x4*>(((n & 1) ? dm2 : dm1) + off) : u32x4{0u, 0u, 0u, 0u};
-      }
-      u32x4 sh[IT], sl[IT];
-#pragma unroll
-      for (int i = 0; i < IT; i++) {
-        const uint32_t off = static_cast<uint32_t>((t0 + wm + 16 * i + lnv) * 2 * nsbp + s0);
-        sh[i] = in ? *reinterpret_cast<const u32x4*>(s16 + off) : u32x4{0u, 0u, 0u, 0u};
-        sl[i] = in ? *reinterpret_cast<const u32x4*>(s16 + off + nsbp) : u32x4{0u, 0u, 0u, 0u};
-      }
-      __builtin_amdgcn_sched_barrier(0);  // every load issued before the first use
-#pragma unroll
-      for (int n = 0; n < NT; n++)
-#pragma unroll
-        for (int d = 0; d < 4; d++) bd[n][d] &= mk[d];
-#pragma unroll
-      for (int i = 0; i < IT; i++) {
-#pragma unroll
-        for (int n = 0; n < NT; n++) {
-          float4v t = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, sh[i]), __builtin_bit_cast(half8, bd[n]),
-                                                             float4v{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-          t = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, sl[i]), __builtin_bit_cast(half8, bd[n]), t, 0, 0, 0);
-#pragma unroll
-          for (int r = 0; r < 4; r++) acc[i][n][r] = __builtin_fmaf(1024.f, t[r], acc[i][n][r]);
-        }
-        __builtin_amdgcn_sched_barrier(0);  // one token group's products at a time
-      }
     }
   }
 
@@ -660,9 +712,15 @@ int sb_launch(const wh::SbGemm& a, hipStream_t s) {
   const dim3 grid(static_cast<unsigned>(SK ? a.sk_g : n_tiles), static_cast<unsigned>(SK ? 1 : a.splits));
   const int upw = SK ? (n_tiles * nsb + a.sk_g - 1) / a.sk_g : 0;
   const int sbps = (nsb + a.splits - 1) / a.splits;
+  // Q4_K's dmin under stream-K: once per tile, by the workgroup that finishes it,
+  // while there are two owners; with more, each part its own, so that what is
+  // handed over and added has the result's size and not the quants' mean's (1536
+  // x 4096 at 804 tokens, error 2.27e-7 -> 2.12e-7; it costs a pass of the table
+  // per part, 1.2 us of 118 at 14336 x 4096 and 512 tokens).
+  const bool parts = 2 * upw <= nsb;
   kernel<<<grid, TWAVES * 64, lds, s>>>(
       a.w, a.w2, a.frag, a.rs, a.bs, a.y, a.n_tokens, a.n_rows, nsb, sbps, tiles_n, n_tiles,
-      a.sk_flags, a.sk_part, upw, a.sk_sub, a.sk_wait, sb_chain(BM, SK ? std::min(nsb, upw) : sbps));
+      a.sk_flags, a.sk_part, upw, a.sk_sub, a.sk_wait, sb_chain(BM, SK ? std::min(nsb, upw) : sbps), parts);
   WH_LAUNCH_CHECK("k-quant gemm kernel launch");
   return WH_OK;
 }
@@ -675,9 +733,12 @@ int sb_launch_bm(const wh::SbGemm& a, hipStream_t s) {
       return a.lo ? sb_launch<TYPE, BM, false, true, true>(a, s) : sb_launch<TYPE, BM, false, true, false>(a, s);
     }
   }
-  if constexpr (TYPE == wh::kGemmQ6S && BM <= 64) {
-    if (sb_lo_first(TYPE, BM, a.n_tokens, (a.k / 256 + a.splits - 1) / a.splits, a.ffn))
+  if (sb_lo_first(TYPE, BM, a.n_tokens, (a.k / 256 + a.splits - 1) / a.splits, a.ffn)) {
+    if constexpr (TYPE == wh::kGemmQ4S) {
+      if constexpr (BM == 128) return sb_launch<TYPE, BM, true, false, true, true>(a, s);
+    } else if constexpr (BM <= 64) {
       return a.lo ? sb_launch<TYPE, BM, false, false, true, true>(a, s) : sb_launch<TYPE, BM, false, false, false, true>(a, s);
+    }
   }
   if (a.ffn) return sb_launch<TYPE, BM, true, false, true>(a, s);
   return a.lo ? sb_launch<TYPE, BM, false, false, true>(a, s) : sb_launch<TYPE, BM, false, false, false>(a, s);
