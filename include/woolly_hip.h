@@ -186,8 +186,9 @@ WH_API int wh_gemv_select(int mode, int* previous);
  *   instead of the [K][N] reshape at lazy_transformer.rs:1091-1101.
  * X is row-major [n_tokens][k] f32, Y is row-major [n_tokens][n_rows] f32.
  * Types: Q4_0, Q4_1, Q8_0 (k % 32 == 0) and Q4_K, Q6_K (k % 256 == 0; with
- * more than 2 tokens the matrix is first rewritten into the workspace as
- * 32-element blocks with f32 scales, the values unchanged).
+ * more than 16 tokens, or fewer on long rows, the matrix is first rewritten
+ * into the workspace, the integer quants and scales unchanged, unless its
+ * handle is prepared).
  * The MFMA path (more than 2 tokens) needs a device workspace of
  * wh_quantized_matmul_workspace_bytes(type, n_rows, k, n_tokens) bytes (256-byte
  * aligned); the call itself never allocates.  WH_ERR_BUFFER_TOO_SMALL if it
@@ -287,10 +288,11 @@ WH_API const void* wh_weight_data(const wh_weight* weight);
 WH_API int wh_weight_info(const wh_weight* weight, int* type, size_t* n_rows, size_t* k,
                           size_t* nbytes);
 /* Converts a Q4_K / Q6_K handle's blocks once, on the stream, into the block
- * layout of the tiled prefill GEMM (the same values: 32-element blocks with
- * f32 scales d * s_j, Q6_K's 16-element halves padded) and keeps that copy
+ * layout of the prefill GEMM (64-element records of the integer quants,
+ * their scales s_j and d; the same values) and keeps that copy
  * with the handle until wh_weight_free; calls of wh_quantized_matmul and
- * wh_ffn_swiglu with more than two tokens whose weight pointer is the
+ * wh_ffn_swiglu that take that GEMM (more than 16 tokens, or fewer on rows
+ * that the several-token kernel does not hold) and whose weight pointer is the
  * handle's data (wh_weight_data) then skip the per-call conversion.  This is
  * the device-side counterpart of the reference's convert-once cache
  * (DequantizationCache::get_or_dequantize,

@@ -5,8 +5,8 @@ The call dispatches on the token count and the shape: one token streams the
 weights once (matrix-core GEMV), 2..16 tokens the several-token GEMV, more
 the tiled MFMA GEMM with 16-, 32-, 64- or 128-token tiles (split-K where the
 tiles are few, stream-K where they would leave CUs idle), a K that is not a
-multiple of 64 the fallback GEMM, and the K-quant formats a conversion to
-32-element blocks first.  The fixed cases of the other tests sit on chosen
+multiple of 64 the fallback GEMM, and the K-quant formats a GEMM of their
+own behind a conversion to stage records.  The fixed cases of the other tests sit on chosen
 shapes; these draw n, k and the token count at random (a fixed seed, so the
 list is the same on every run) around each of those thresholds, rows that
 are not a multiple of 16 or 256 included, and check sampled tokens

@@ -185,8 +185,9 @@ def owners_cases():
 @pytest.mark.parametrize("n,k,m", owners_cases())
 def test_stream_k_fallback_matmul(gpu, orc, t, n, k, m):
     """Wait bound 0: the finishing workgroup computes the rest of each shared
-    tile in a second pass (for Q4_K also the dmin term of every super-block);
-    the result is the product within the same bars."""
+    tile in a second pass (for Q4_K also the dmin term of every super-block;
+    Q4_K shares tiles in the first shape only, test_stream_k_kquant_parts has
+    more); the result is the product within the same bars."""
     print(f"[case] stream-K fallback matmul type={t} m={m} n={n} k={k}", flush=True)
     w = synth.quantized_weight(t, n, k, seed=n + k + t)
     x = synth.activations(m * k, seed=m + t).reshape(m, k)

@@ -1,5 +1,5 @@
 // gemm_dev.hpp -- device helpers shared by the prefill GEMMs (gemm_tiled.hip,
-// gemm_sb.hip): MFMA operand types, global -> LDS copies, the waits on them and
+// gemm_sb.hpp): MFMA operand types, global -> LDS copies, the waits on them and
 // the stream-K partial tiles.
 #pragma once
 
@@ -76,14 +76,13 @@ __device__ __forceinline__ int __attribute__((ext_vector_type(4))) sk_rsrc(const
   return r;
 }
 
-// Waits until at most min(n, J) stages of N copies each are in flight (and the
-// X operations issued behind them).
-template <int N, int J, int X = 0>
+// Waits until at most min(n, J) stages of N copies each are in flight.
+template <int N, int J>
 __device__ __forceinline__ void wait_stages(int n) {
   if constexpr (J == 0) {
-    wait_vmcnt<X>();
+    wait_vmcnt<0>();
   } else {
-    if (n >= J) wait_vmcnt<J * N + X>();
-    else wait_stages<N, J - 1, X>(n);
+    if (n >= J) wait_vmcnt<J * N>();
+    else wait_stages<N, J - 1>(n);
   }
 }

@@ -37,7 +37,8 @@
 // weights are formed right after its last MFMA, so no phase starts with a
 // burst of LDS reads (the bound of gemm_tiled.hip's schedule after the VALU).
 // The barrier of a stage stands behind the last LDS read of its slot, in the
-// middle of its second step.
+// middle of its second step.  LF (sb_lo_first): the same with the two steps'
+// products in another order, both steps' operands in registers.
 #pragma once
 
 #include "gemm_dev.hpp"
@@ -58,16 +59,17 @@ template <int TYPE>
 constexpr int sb_rec() { return TYPE == wh::kGemmQ4S ? 40 : 80; }  // bytes per row and stage
 
 // Stages after the first that the matrix cores accumulate before d is applied
-// (0: 64 elements, 1: 128), for the sb super-blocks that a workgroup
-// sums per tile.  An MFMA rounds its
-// products at the size of its C operand, so a long chain loses more than the f32
-// FMAs of a short one; in a long sum the FMAs do, since the sum outgrows the
-// chain.  A step's products with an x_lo or w_lo come first, while C is small.
-// Error against 64 bits, Q4_K 14336 x 4096: chains of 256, x_hi first, 2.8e-7
-// at M=32, 2.9e-7 at M=128, 3.0e-7 at M=512; of 64, x_lo first, 2.0e-7, 2.3e-7,
-// 2.7e-7; of 128 2.4e-7 at M=128, 2.6e-7 at M=512 (a workgroup
-// sums 4 super-blocks at M=128, 14 at M=512).  Of 32 worse again: 2.2e-7 at M=32.  Time at M=512: 127
-// us with 64, 120.6 with 128; at M=128 55.1 and 53.5.
+// (0: 64 elements, 1: 128), for the sb super-blocks that a workgroup sums per
+// tile.  An MFMA rounds its products at the size of its C operand, so a long
+// chain loses more than the f32 FMAs of a short one; in a long sum the FMAs do,
+// since the sum outgrows the chain.  Against 64 bits, Q4_K 14336 x 4096: chains
+// of 256 elements 2.8e-7 at M=32, 3.0e-7 at M=512; of 64 2.0e-7 and 2.7e-7; of 128
+// 2.6e-7 at M=512 (14 super-blocks); of 32 2.2e-7 at M=32.  From 8 super-blocks on,
+// in 12 shapes of 8 to 28 and both types, 128 elements took 0.94 to 0.97 of the time
+// of 64 (M=512 14336 x 4096 Q4_K 127.3 -> 121.5 us, Q6_K 169.2 -> 162.4) and are
+// nearer for Q4_K (14336 x 4096 2.66e-7 -> 2.57e-7, 4096 x 14336 3.02e-7 -> 2.71e-7)
+// and for Q6_K from 14 on (4096 x 14336 1.85e-7 -> 1.69e-7); Q6_K loses up to 3% at 8
+// to 12 (8192 x 2048 1.40e-7 -> 1.44e-7; 2.08e-7 with 16-element blocks).
 inline int sb_chain(int bm, int sb) { return bm == 128 && sb >= 8 ? 1 : 0; }
 
 // Q6_K where a workgroup sums one or two super-blocks, and the 64-token tiles of

@@ -1050,7 +1050,7 @@ bool gemm_tiled_ok(int type, const void* w, const float* x, size_t n_rows, size_
     case WH_TYPE_Q4_0: lds = lds_typed<WH_TYPE_Q4_0>(b); break;
     case WH_TYPE_Q4_1: lds = lds_typed<WH_TYPE_Q4_1>(b); break;
     case WH_TYPE_Q8_0: lds = lds_typed<WH_TYPE_Q8_0>(b); break;
-    default: lds = static_cast<size_t>(160) * 1024; break;  // gemm_sb.hpp: a ring in all of the LDS
+    default: lds = static_cast<size_t>(160) * 1024; break;  // gemm_sb.hpp: three stages, up to 156 KB
   }
   return lds <= max_lds_per_block();
 }
