@@ -234,6 +234,9 @@ def test_kquant_split_k_has_no_empty_planes(t, nsb, planes):
     (14336, 8192, 100, 4, 4),                                 # seven super-blocks of eight: split-K
     (10240, 5632, 100, 0, 0), (20480, 4096, 100, 0, 0),       # four of six, five of eight: stream-K
     (28672, 4096, 100, 0, 0),                                 # two splits: seven of eight too
+    (8192, 2048, 512, 0, 0), (30720, 4096, 100, 0, 0),        # and half tiles
+    (4096, 14336, 512, 0, 0),                                 # a quarter of a tile on each CU
+    (14336, 4096, 100, 4, 4),                                 # a quarter of a tile on 224 of them
     (16384, 2048, 60, 0, 0), (14336, 4096, 512, 0, 0)])       # 64-token tiles; without split-K
 def test_kquant_stream_k_or_split_k(n, k, m, q4k, q6k):
     """The workspace shows which the plan takes: split-K planes, or (0 here) a

@@ -883,20 +883,25 @@ int sk_grid(size_t n_tiles, size_t tile_st) {
 // their parts over one after the other, so with more than four, stream-K loses
 // to split-K planes and a reduce (100 tokens, Q4_K, stream-K / split-K in us:
 // 5 tiles of 56 super-blocks 77.3 / 53.4, 16 of 32 56.0 / 42.4, 32 of 22 54.4 /
-// 47.1, 32 of 56 85.2 / 81.1).  With up to four it wins where it shortens the
-// longest workgroup by more than an eighth (40 of 22, four super-blocks instead
-// of six: 56.1 / 62.9; 80 of 16, five of eight: 64.8 / 73.3), and not below that
-// (56 of 32, seven of eight: 84.2 / 77.4; 64 of 22, six of six: 73.9 / 69.5).
-// 64-token tiles hand over half as much: they gain with up to four in any case
-// (60 tokens, 64 of 8: 27.0 / 28.8; 64 of 22 47.1 / 45.6).  Against one or two
-// splits it needs any shortening (100 tiles of 13, six of seven: 68.9 / 72.2; 112
-// of 16, seven of eight: 73.4 / 74.0).
+// 47.1).  With four it wins where it shortens the longest workgroup by more than
+// an eighth (40 of 22, four super-blocks instead of six: 57.7 / 63.9; 48 of 32, six
+// of eight: 73.8 / 75.1) and not below that (56 of 32, seven of eight: 83.3 / 77.0;
+// 64 of 22, six of six: 70.9 / 67.4), unless every CU has exactly one part (512
+// tokens: 64 of 32 84.7 / 86.8).  With two any shortening will do (100 of 13, six of
+// seven: 68.1 / 73.1), or parts that are a whole fraction of a tile (512 tokens: 128
+// of 8 53.2 / 58.0).  64-token tiles hand over half as much: they gain with up to
+// four in any case (60 tokens, 64 of 8: 27.0 / 28.8; 64 of 22 47.1 / 45.6).  Without
+// split-K it needs any shortening.
 int sb_sk_grid(size_t n_tiles, size_t nsb, int bm, int splits) {
   const size_t g = static_cast<size_t>(wh::cu_count());
   if (g == 0 || g % 8 != 0 || n_tiles % g == 0 || bm < 64 || splits > 4) return 0;
   const size_t upw = (n_tiles * nsb + g - 1) / g;
   const size_t per = (n_tiles * splits + g - 1) / g * ((nsb + splits - 1) / splits);
-  const bool gain = splits <= 2 ? upw < per : bm == 64 || 8 * upw < 7 * per;
+  const bool whole = nsb % upw == 0;
+  bool gain;
+  if (splits == 1) gain = upw < per;
+  else if (splits == 2) gain = bm == 64 || upw < per || whole;
+  else gain = bm == 64 || 8 * upw < 7 * per || (whole && n_tiles * splits == g);
   return upw >= 2 && gain ? static_cast<int>(g) : 0;
 }
 
