@@ -110,15 +110,17 @@ def test_stream_k_kquant_matmul(gpu, orc, t, n, k, m):
 
 
 # (n, k, m), super-blocks per workgroup of a tile's: 80 tiles 5 of 16, 40 tiles 4 of
-# 22, 64 tiles of 64 tokens 2 of 8 and 8 of 32, 168 tiles 11 of 16
-KQ_PARTS = [(20480, 4096, 100), (10240, 5632, 100), (16384, 2048, 60), (16384, 8192, 60), (14336, 4096, 300)]
+# 22, 64 tiles of 64 tokens 2 of 8 and 8 of 32, 168 tiles 11 of 16, 36 tiles 2 of 13
+# and 128 tiles 4 of 8
+KQ_PARTS = [(20480, 4096, 100), (10240, 5632, 100), (16384, 2048, 60), (16384, 8192, 60), (14336, 4096, 300),
+            (2304, 3328, 500), (8192, 2048, 512)]
 
 
 @pytest.mark.parametrize("t", [Q4_K, Q6_K])
 @pytest.mark.parametrize("n,k,m", KQ_PARTS)
 @pytest.mark.parametrize("wait", [None, 0])
 def test_stream_k_kquant_parts(gpu, orc, t, n, k, m, wait):
-    """K-quant tiles of 64 and 128 tokens with up to six owners, handed over or
+    """K-quant tiles of 64 and 128 tokens with two to seven owners, handed over or
     (wait bound 0) computed by the finishing workgroup in a second pass.  Q4_K:
     dmin of -128 to -512 d, against activations with a mean of 0.5, carries most of
     each output, so a part's end inside the 32-super-block windows shows."""

@@ -124,7 +124,7 @@ __global__ __launch_bounds__(TWAVES * 64, 1) void gemm_sb_kernel(
     const float* __restrict__ rscale, const float* __restrict__ bsum, float* __restrict__ y, int n_tokens, int n_rows,
     int nsb, int sb_per_split, int tiles_n, int n_tiles, uint32_t* __restrict__ sk_flags, float* __restrict__ sk_part,
     int sk_upw, int sk_sub, uint32_t sk_wait,
-    int chain, bool parts) {
+    int chain) {
   using C = SbCfg<BM>;
   using S = SbStage<TYPE, BM, LO>;
   constexpr int IT = C::IT, NT = C::NT, REC = sb_rec<TYPE>(), N = S::N;
@@ -306,10 +306,80 @@ __global__ __launch_bounds__(TWAVES * 64, 1) void gemm_sb_kernel(
   for (int i = 0; i < IT; i++)
 #pragma unroll
     for (int n = 0; n < NT; n++) acc[i][n] = float4v{0.f, 0.f, 0.f, 0.f};
+  // dmin: acc += dmin[row][sb] S[token][sb] over super-blocks [sb_lo, sb_hi), as
+  // matrix-core products over windows of 32: lane group g holds super-blocks
+  // 8g .. 8g + 7 of the window in both operands (B: the fp16 table behind the
+  // records, those outside masked to zero; A: the packing's sums as hi + lo fp16
+  // limbs of S 2^-10).
+  auto add_dmin = [&](int sb_lo, int sb_hi) {
+    const int nsbp = (nsb + 7) & ~7;
+    const size_t table = static_cast<size_t>(nsb) * 4 * stage_stride;
+    const uint16_t* dm1 = reinterpret_cast<const uint16_t*>(W + table);
+    const uint16_t* dm2 = FFNP ? reinterpret_cast<const uint16_t*>(W2 + table) : dm1;
+    const uint16_t* s16 = reinterpret_cast<const uint16_t*>(bsum);
+    // opaque, so that the loads' offsets are formed here and not held in
+    // registers through the stage loop
+    int lnv = ln;
+    asm volatile("" : "+v"(lnv));
+    for (int w0 = sb_lo & ~31; w0 < sb_hi; w0 += 32) {
+      const int s0 = w0 + 8 * g;
+      const bool in = s0 < nsbp;
+      uint32_t mk[4];
+#pragma unroll
+      for (int d = 0; d < 4; d++) {
+        const int a = s0 + 2 * d;
+        mk[d] = (a >= sb_lo && a < sb_hi ? 0x0000FFFFu : 0u) | (a + 1 >= sb_lo && a + 1 < sb_hi ? 0xFFFF0000u : 0u);
+      }
+      u32x4 bd[NT];
+#pragma unroll
+      for (int n = 0; n < NT; n++) {
+        const int row = r0 + (FFNP ? wn / 2 + 16 * (n >> 1) : wn + 16 * n) + lnv;
+        const uint32_t off = static_cast<uint32_t>(min(row, n_rows - 1) * nsbp + s0);
+        bd[n] = in ? *reinterpret_cast<const u32x4*>(((n & 1) ? dm2 : dm1) + off) : u32x4{0u, 0u, 0u, 0u};
+      }
+      u32x4 sh[IT], sl[IT];
+#pragma unroll
+      for (int i = 0; i < IT; i++) {
+        const uint32_t off = static_cast<uint32_t>((t0 + wm + 16 * i + lnv) * 2 * nsbp + s0);
+        sh[i] = in ? *reinterpret_cast<const u32x4*>(s16 + off) : u32x4{0u, 0u, 0u, 0u};
+        sl[i] = in ? *reinterpret_cast<const u32x4*>(s16 + off + nsbp) : u32x4{0u, 0u, 0u, 0u};
+      }
+      __builtin_amdgcn_sched_barrier(0);  // every load issued before the first use
+#pragma unroll
+      for (int n = 0; n < NT; n++)
+#pragma unroll
+        for (int d = 0; d < 4; d++) bd[n][d] &= mk[d];
+#pragma unroll
+      for (int i = 0; i < IT; i++) {
+#pragma unroll
+        for (int n = 0; n < NT; n++) {
+          float4v t = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, sh[i]), __builtin_bit_cast(half8, bd[n]),
+                                                             float4v{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+          t = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, sl[i]), __builtin_bit_cast(half8, bd[n]), t, 0, 0, 0);
+#pragma unroll
+          for (int r = 0; r < 4; r++) acc[i][n][r] = __builtin_fmaf(1024.f, t[r], acc[i][n][r]);
+        }
+        __builtin_amdgcn_sched_barrier(0);  // one token group's products at a time
+      }
+    }
+  };
+  // Stream-K: 128-token tiles add it over all of the tile, in the workgroup that
+  // finishes it; in parts of up to three super-blocks, of which a tile has five or
+  // more, and in 64-token tiles, each part its own (own_dmin), so that what is
+  // handed over has the result's size and not the quants' mean's (1536 x 4096 at 804
+  // tokens, error 2.27e-7 -> 2.15e-7, 53.6 us either way; it costs a pass of the
+  // table per part: 10240 x 5632 at 100 tokens, four super-blocks each, 56.1 -> 57.2
+  // us).  64-token tiles add it before they wait for the other parts, for which the
+  // 128-token kernel has no registers.
+  constexpr bool EARLY = SK && BM < 128;
+  const bool own_dmin = !SK || EARLY || sk_upw <= 3;
   // A head part (SK) that does not get every other owner's slot in time runs
   // a second pass over the rest of the tile, into the same accumulators.
+  int done = sb_b;  // end of the super-blocks summed here
+#pragma unroll 1
   for (int pass = 0; pass < 2; pass++) {
   const int sb0 = pass ? sb_b : sb_a;
+  if (pass > 0) done = nsb;
   const int n_stages = 4 * ((pass ? nsb : sb_b) - sb0);
   if (pass > 0) __syncthreads();  // the ring of the first pass is no longer read
   to_issue = n_stages;
@@ -550,65 +620,7 @@ __global__ __launch_bounds__(TWAVES * 64, 1) void gemm_sb_kernel(
       cur = nxt;
   }
   apply(NT - 1, dn[NT - 1]);
-  if constexpr (Q4) {
-    // dmin: acc += dmin[row][sb] S[token][sb] over the super-blocks just summed
-    // (stream-K: see sb_launch), as matrix-core products over windows of 32 super-blocks: lane group g
-    // holds super-blocks 8g .. 8g + 7 of the window in both operands (B: the
-    // fp16 table behind the records, those of other splits masked to zero; A:
-    // the packing's sums as hi + lo fp16 limbs of S 2^-10).
-    const int nsbp = (nsb + 7) & ~7;
-    const bool own = !SK || parts;
-    const int sb_lo = own ? sb0 : 0, sb_hi = own ? (pass ? nsb : sb_b) : (pass == 0 && sb_a == 0 ? nsb : 0);
-    const size_t table = static_cast<size_t>(nsb) * 4 * stage_stride;
-    const uint16_t* dm1 = reinterpret_cast<const uint16_t*>(W + table);
-    const uint16_t* dm2 = FFNP ? reinterpret_cast<const uint16_t*>(W2 + table) : dm1;
-    const uint16_t* s16 = reinterpret_cast<const uint16_t*>(bsum);
-    // opaque, so that the loads' offsets are formed here and not held in
-    // registers through the stage loop
-    int lnv = ln;
-    asm volatile("" : "+v"(lnv));
-    for (int w0 = sb_lo & ~31; w0 < sb_hi; w0 += 32) {
-      const int s0 = w0 + 8 * g;
-      const bool in = s0 < nsbp;
-      uint32_t mk[4];
-#pragma unroll
-      for (int d = 0; d < 4; d++) {
-        const int a = s0 + 2 * d;
-        mk[d] = (a >= sb_lo && a < sb_hi ? 0x0000FFFFu : 0u) | (a + 1 >= sb_lo && a + 1 < sb_hi ? 0xFFFF0000u : 0u);
-      }
-      u32x4 bd[NT];
-#pragma unroll
-      for (int n = 0; n < NT; n++) {
-        const int row = r0 + (FFNP ? wn / 2 + 16 * (n >> 1) : wn + 16 * n) + lnv;
-        const uint32_t off = static_cast<uint32_t>(min(row, n_rows - 1) * nsbp + s0);
-        bd[n] = in ? *reinterpret_cast<const u32x4*>(((n & 1) ? dm2 : dm1) + off) : u32x4{0u, 0u, 0u, 0u};
-      }
-      u32x4 sh[IT], sl[IT];
-#pragma unroll
-      for (int i = 0; i < IT; i++) {
-        const uint32_t off = static_cast<uint32_t>((t0 + wm + 16 * i + lnv) * 2 * nsbp + s0);
-        sh[i] = in ? *reinterpret_cast<const u32x4*>(s16 + off) : u32x4{0u, 0u, 0u, 0u};
-        sl[i] = in ? *reinterpret_cast<const u32x4*>(s16 + off + nsbp) : u32x4{0u, 0u, 0u, 0u};
-      }
-      __builtin_amdgcn_sched_barrier(0);  // every load issued before the first use
-#pragma unroll
-      for (int n = 0; n < NT; n++)
-#pragma unroll
-        for (int d = 0; d < 4; d++) bd[n][d] &= mk[d];
-#pragma unroll
-      for (int i = 0; i < IT; i++) {
-#pragma unroll
-        for (int n = 0; n < NT; n++) {
-          float4v t = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, sh[i]), __builtin_bit_cast(half8, bd[n]),
-                                                             float4v{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-          t = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, sl[i]), __builtin_bit_cast(half8, bd[n]), t, 0, 0, 0);
-#pragma unroll
-          for (int r = 0; r < 4; r++) acc[i][n][r] = __builtin_fmaf(1024.f, t[r], acc[i][n][r]);
-        }
-        __builtin_amdgcn_sched_barrier(0);  // one token group's products at a time
-      }
-    }
-  }
+  if constexpr (Q4 && EARLY) add_dmin(sb0, done);
   if constexpr (!SK) break;
   if (pass > 0 || sb_a > 0 || sb_b == nsb) break;  // a tail part, the whole tile, or done here
   // head part: wait for the owners of the rest of the tile, then add their slots in order
@@ -643,6 +655,9 @@ __global__ __launch_bounds__(TWAVES * 64, 1) void gemm_sb_kernel(
   }
   // otherwise: the rest of the tile, here
   }  // pass
+  if constexpr (Q4 && !EARLY)
+    if (own_dmin || sb_a == 0) add_dmin(sb_a, own_dmin ? done : nsb);
+
   if constexpr (SK) {
     if (sb_a > 0) {
       // a tail part: the raw accumulators to this workgroup's slot, then its flag
@@ -714,15 +729,9 @@ int sb_launch(const wh::SbGemm& a, hipStream_t s) {
   const dim3 grid(static_cast<unsigned>(SK ? a.sk_g : n_tiles), static_cast<unsigned>(SK ? 1 : a.splits));
   const int upw = SK ? (n_tiles * nsb + a.sk_g - 1) / a.sk_g : 0;
   const int sbps = (nsb + a.splits - 1) / a.splits;
-  // Q4_K's dmin under stream-K: once per tile, by the workgroup that finishes it,
-  // while there are two owners; with more, each part its own, so that what is
-  // handed over and added has the result's size and not the quants' mean's (1536
-  // x 4096 at 804 tokens, error 2.27e-7 -> 2.12e-7; it costs a pass of the table
-  // per part, 1.2 us of 118 at 14336 x 4096 and 512 tokens).
-  const bool parts = 2 * upw <= nsb;
   kernel<<<grid, TWAVES * 64, lds, s>>>(
       a.w, a.w2, a.frag, a.rs, a.bs, a.y, a.n_tokens, a.n_rows, nsb, sbps, tiles_n, n_tiles,
-      a.sk_flags, a.sk_part, upw, a.sk_sub, a.sk_wait, sb_chain(BM, SK ? std::min(nsb, upw) : sbps), parts);
+      a.sk_flags, a.sk_part, upw, a.sk_sub, a.sk_wait, sb_chain(BM, SK ? std::min(nsb, upw) : sbps));
   WH_LAUNCH_CHECK("k-quant gemm kernel launch");
   return WH_OK;
 }
