@@ -113,7 +113,7 @@ __global__ __launch_bounds__(256) void kq_dequant_kernel(const uint8_t* __restri
         *reinterpret_cast<float4*>(out + e) = make_float4(v[0], v[1], v[2], v[3]);
       } else {
         kq_quad<TYPE>(data + b * kq_bytes<TYPE>(), lane, v);
-        if (OUT16 && e + 4 <= n) {
+        if (OUT16 && !WIDE && e + 4 <= n) {  // (WIDE: the matrix's last block only)
           *reinterpret_cast<float4*>(out + e) = make_float4(v[0], v[1], v[2], v[3]);
         } else {
           for (int t = 0; t < 4 && e + t < n; t++) out[e + t] = v[t];
